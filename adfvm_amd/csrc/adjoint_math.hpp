@@ -60,214 +60,223 @@ template <typename T> ADFVM_HD void conservative_vjp(const Phys<T>& ph, const T*
     wb[3] += eb * ph.Cv;
 }
 
-// reconstruct (one side): out = clamp(wC + (wD-wC)*lw + qw.g)
+// Which value each of reconstruct()'s five results is, two bits each: 0 the
+// reconstructed value, 1 clamped to the cell's own value, 2 to the other
+// cell's.  Kept in place of the inputs, so that these need not stay in
+// registers until the reverse of the reconstruction.
 template <typename T>
-ADFVM_HD void reconstruct_vjp(const T* wC, const T* gC, const T* wD, T lw, const T* qw, const T* ob,
-                              int limit, T* wCb, T* gCb, T* wDb) {
+ADFVM_HD int reconstruct_taken(const T* wC, const T* gC, const T* wD, T lw, const T* qw) {
+    int taken = 0;
     for (int i = 0; i < 5; i++) {
-        T b = ob[i];
-        if (limit) {
-            const T* g = gC + 3 * i;
-            T v = wC[i] + (wD[i] - wC[i]) * lw + (qw[0] * g[0] + qw[1] * g[1] + qw[2] * g[2]);
-            T lo = wC[i] < wD[i] ? wC[i] : wD[i];
-            T hi = wC[i] < wD[i] ? wD[i] : wC[i];
-            // out = v < lo ? lo : (v > hi ? hi : v), lo/hi selected as in
-            // reconstruct(); the adjoint follows the selected value
-            if (v < lo) {
-                if (wC[i] < wD[i]) wCb[i] += b; else wDb[i] += b;
-                continue;
-            }
-            if (v > hi) {
-                if (wC[i] < wD[i]) wDb[i] += b; else wCb[i] += b;
-                continue;
-            }
+        const T* g = gC + 3 * i;
+        T v = wC[i] + (wD[i] - wC[i]) * lw + (qw[0] * g[0] + qw[1] * g[1] + qw[2] * g[2]);
+        const bool up = wC[i] < wD[i];
+        const T lo = up ? wC[i] : wD[i], hi = up ? wD[i] : wC[i];
+        // out = v < lo ? lo : (v > hi ? hi : v), as in reconstruct()
+        if (v < lo) taken |= (up ? 1 : 2) << (2 * i);
+        else if (v > hi) taken |= (up ? 2 : 1) << (2 * i);
+    }
+    return taken;
+}
+
+// reconstruct (one side): out = clamp(wC + (wD-wC)*lw + qw.g); the adjoint
+// follows the selected value
+template <typename T>
+ADFVM_HD void reconstruct_vjp(T lw, const T* qw, const T* ob, int taken, T* wCb, T* gCb, T* wDb) {
+    if (taken == 0) {
+        for (int i = 0; i < 5; i++) {
+            const T d = ob[i] * lw;
+            wCb[i] += ob[i] - d;
+            wDb[i] += d;
+            for (int k = 0; k < 3; k++) gCb[3 * i + k] += ob[i] * qw[k];
         }
-        wCb[i] += b * (T(1) - lw);
-        wDb[i] += b * lw;
+        return;
+    }
+    for (int i = 0; i < 5; i++) {
+        const int which = (taken >> (2 * i)) & 3;
+        const T b = which == 0 ? ob[i] : T(0), d = b * lw;
+        wCb[i] += which == 1 ? ob[i] : b - d;
+        wDb[i] += which == 2 ? ob[i] : d;
         for (int k = 0; k < 3; k++) gCb[3 * i + k] += b * qw[k];
     }
 }
 
-// Roe flux reverse.  Inputs used: U (w[0..2]), p (w[4]), rho (q[0]).
+// One side of a Roe face from its primitive values: total enthalpy h =
+// g/(g-1) p/rho + |U|^2/2 = g Cv T + |U|^2/2, R = (g-1) Cv.
+template <typename T> struct RoeSide {
+    T Un, iRT, rho, h, s;        // U.n, 1/(R T), density, total enthalpy, sqrt(rho)
+    T c, Ue;                     // sound speed and U.n as the entropy fix compares them
+};
+// FP32: density p/(R T) and sound speed sqrt(g R T) by the one reciprocal.
+ADFVM_HD void roe_density(const Phys<float>& ph, const float* w, RoeSide<float>& o) {
+    const float RT = (ph.gamma - 1.0f) * ph.Cv * w[3];
+    o.iRT = recip(RT);
+    o.rho = w[4] * o.iRT;
+    o.c = fsqrt(ph.gamma * RT);
+    o.Ue = o.Un;
+}
+// Otherwise in the reference's own terms (riemann.py:31-58: c = sqrt(g p/rho),
+// U.n as (rho U.n)/rho): where a side's value equals the other's up to
+// rounding, as in a field of uniform temperature, the sign that rounding
+// gives the difference decides the branch of the adjoint.
+template <typename T> ADFVM_HD void roe_density(const Phys<T>& ph, const T* w, RoeSide<T>& o) {
+    o.iRT = recip((ph.gamma - T(1)) * ph.Cv * w[3]);
+    o.rho = w[4] / (ph.Cv * w[3] * (ph.gamma - T(1)));
+    o.c = fsqrt(ph.gamma * w[4] / o.rho);
+    o.Ue = o.rho * o.Un / o.rho;
+}
+template <typename T> ADFVM_HD void roe_side(const Phys<T>& ph, const T* w, const T* n, RoeSide<T>& o) {
+    o.Un = w[0] * n[0] + w[1] * n[1] + w[2] * n[2];
+    roe_density(ph, w, o);
+    o.h = ph.gamma * ph.Cv * w[3] + T(0.5) * (w[0] * w[0] + w[1] * w[1] + w[2] * w[2]);
+    o.s = fsqrt(o.rho);
+}
+
+// The Roe averages, jumps and dissipation of a face (riemann.eulerRoe,
+// adFVM/riemann.py:21-70).  stabilise(eps) = eps + SMALL for eps >= 0 (adpy's
+// definition is not in the reference).
+template <typename T> struct RoeFace {
+    T idv, a, b;                 // 1/(sL + sR) and the sides' weights sL, sR over their sum
+    T U[3], h, q, c, ic, Un;     // averages: velocity, enthalpy, |U|^2/2, sound speed, 1/c, normal velocity
+    T drho, drhoU[3], drhoE;
+    T ieps, r1, r2, r3;          // 1/eps; eigenvalues over eps
+    bool f1, f2, f3;             // eigenvalues inside the entropy fix
+    T l1;                        // fixed |Un|
+    T m2, m3;                    // (l2 - l3)/2, (l2 + l3)/2 - l1
+    T x, y;                      // pressure jump over c, -rho U.n jump
+    T k6, s6, s7;                // m3 x - m2 y; s6 = k6/c; s7 = m3 y - m2 x
+};
 template <typename T>
-ADFVM_HD void roe_flux_vjp(const Phys<T>& ph, const T* wL, const T* qL, const T* wR, const T* qR, const T* n,
-                           const T* Fb, T* wLb, T* qLb, T* wRb, T* qRb) {
-    const T g = ph.gamma, gm1 = ph.gamma - T(1);
-    const T *UL = wL, *UR = wR;
-    T pL = wL[4], pR = wR[4], rhoL = qL[0], rhoR = qR[0];
-    // ---- forward recompute
-    T UnL = UL[0] * n[0] + UL[1] * n[1] + UL[2] * n[2];
-    T UnR = UR[0] * n[0] + UR[1] * n[1] + UR[2] * n[2];
-    T rhoUnL = rhoL * UnL, rhoUnR = rhoR * UnR;
-    T hL = g * pL / (gm1 * rhoL) + T(0.5) * (UL[0] * UL[0] + UL[1] * UL[1] + UL[2] * UL[2]);
-    T hR = g * pR / (gm1 * rhoR) + T(0.5) * (UR[0] * UR[0] + UR[1] * UR[1] + UR[2] * UR[2]);
-    T sL = fsqrt(rhoL), sR = fsqrt(rhoR);
-    T dv = sL + sR;
-    T UF[3];
-    for (int i = 0; i < 3; i++) UF[i] = (UL[i] * sL + UR[i] * sR) / dv;
-    T hF = (hL * sL + hR * sR) / dv;
-    T qF = T(0.5) * (UF[0] * UF[0] + UF[1] * UF[1] + UF[2] * UF[2]);
-    T a2F = gm1 * (hF - qF);
-    T aF = fsqrt(a2F);
-    T UnF = UF[0] * n[0] + UF[1] * n[1] + UF[2] * n[2];
-    T drho = rhoR - rhoL;
-    T drhoU[3];
-    for (int i = 0; i < 3; i++) drhoU[i] = rhoR * UR[i] - rhoL * UL[i];
-    T drhoE = (hR * rhoR - pR) - (hL * rhoL - pL);
-    T lam1 = fabs_(UnF), lam2 = fabs_(UnF + aF), lam3 = fabs_(UnF - aF);
-    T cL = fsqrt(g * pL / rhoL), cR = fsqrt(g * pR / rhoR);
-    T ea = rhoUnL / rhoL - rhoUnR / rhoR;
-    T eb_ = cL - cR;
-    T eps = T(0.5) * fabs_(ea);
-    eps += T(0.5) * fabs_(eb_);
-    eps = eps < T(0) ? eps - ph.small : eps + ph.small;
-    T e2 = T(2) * eps;
-    bool f1 = lam1 < e2, f2 = lam2 < e2, f3 = lam3 < e2;
-    T l1 = f1 ? T(0.25) * lam1 * lam1 / eps + eps : lam1;
-    T l2 = f2 ? T(0.25) * lam2 * lam2 / eps + eps : lam2;
-    T l3 = f3 ? T(0.25) * lam3 * lam3 / eps + eps : lam3;
-    T abv1 = T(0.5) * (l2 + l3);
-    T abv2 = T(0.5) * (l2 - l3);
-    T abv3 = abv1 - l1;
-    T abv4 = gm1 * (qF * drho - (UF[0] * drhoU[0] + UF[1] * drhoU[1] + UF[2] * drhoU[2]) + drhoE);
-    T abv5 = UnF * drho - (drhoU[0] * n[0] + drhoU[1] * n[1] + drhoU[2] * n[2]);
-    T abv6 = abv3 * abv4 / a2F - abv2 * abv5 / aF;
-    T abv7 = abv3 * abv5 - abv2 * abv4 / aF;
-    (void)abv1;
-    // ---- reverse
-    T l1b = 0, drhob = 0, abv6b = 0, abv7b = 0, drhoEb = 0, hFb = 0, UnFb = 0;
-    T drhoUb[3] = {0, 0, 0}, UFb[3] = {0, 0, 0}, FU0b[3];
-    T Fr0b = Fb[0];
-    l1b += -T(0.5) * Fb[0] * drho;
-    drhob += -T(0.5) * Fb[0] * l1;
-    abv6b += -T(0.5) * Fb[0];
+ADFVM_HD void roe_face(const Phys<T>& ph, const T* wL, const RoeSide<T>& L, const T* wR, const RoeSide<T>& R,
+                       const T* n, RoeFace<T>& o) {
+    const T gm1 = ph.gamma - T(1);
+    o.idv = recip(L.s + R.s);
+    o.a = L.s * o.idv;
+    o.b = R.s * o.idv;
+    for (int i = 0; i < 3; i++) o.U[i] = wL[i] * o.a + wR[i] * o.b;
+    o.h = L.h * o.a + R.h * o.b;
+    o.q = T(0.5) * (o.U[0] * o.U[0] + o.U[1] * o.U[1] + o.U[2] * o.U[2]);
+    o.c = fsqrt(gm1 * (o.h - o.q));
+    o.ic = recip(o.c);
+    o.Un = o.U[0] * n[0] + o.U[1] * n[1] + o.U[2] * n[2];
+    o.drho = R.rho - L.rho;
+    for (int i = 0; i < 3; i++) o.drhoU[i] = R.rho * wR[i] - L.rho * wL[i];
+    o.drhoE = (R.h * R.rho - wR[4]) - (L.h * L.rho - wL[4]);
+    const T lam1 = fabs_(o.Un), lam2 = fabs_(o.Un + o.c), lam3 = fabs_(o.Un - o.c);
+    T eps = T(0.5) * fabs_(L.Ue - R.Ue);
+    eps += T(0.5) * fabs_(L.c - R.c);
+    eps = eps + ph.small;
+    o.ieps = recip(eps);
+    const T e2 = T(2) * eps;
+    o.f1 = lam1 < e2; o.f2 = lam2 < e2; o.f3 = lam3 < e2;
+    o.r1 = lam1 * o.ieps; o.r2 = lam2 * o.ieps; o.r3 = lam3 * o.ieps;
+    o.l1 = o.f1 ? T(0.25) * lam1 * o.r1 + eps : lam1;
+    const T l2 = o.f2 ? T(0.25) * lam2 * o.r2 + eps : lam2;
+    const T l3 = o.f3 ? T(0.25) * lam3 * o.r3 + eps : lam3;
+    o.m2 = T(0.5) * (l2 - l3);
+    o.m3 = T(0.5) * (l2 + l3) - o.l1;
+    o.x = gm1 * (o.q * o.drho - (o.U[0] * o.drhoU[0] + o.U[1] * o.drhoU[1] + o.U[2] * o.drhoU[2]) + o.drhoE) * o.ic;
+    o.y = o.Un * o.drho - (o.drhoU[0] * n[0] + o.drhoU[1] * n[1] + o.drhoU[2] * n[2]);
+    o.k6 = o.m3 * o.x - o.m2 * o.y;
+    o.s6 = o.k6 * o.ic;
+    o.s7 = o.m3 * o.y - o.m2 * o.x;
+}
+
+// Reverse of one side's derived values: adds the adjoints of U, T, p from
+// those of Un, rho, h and c (s goes through rho).
+template <typename T>
+ADFVM_HD void roe_side_vjp(const Phys<T>& ph, const T* w, const T* n, const RoeSide<T>& o, T Unb, T rhob, T hb, T cb,
+                           T* wb) {
+    const T RiRT = (ph.gamma - T(1)) * ph.Cv * o.iRT;         // 1/T
+    for (int i = 0; i < 3; i++) wb[i] += Unb * n[i] + hb * w[i];
+    wb[3] += ph.gamma * ph.Cv * hb + (T(0.5) * cb * o.c - rhob * o.rho) * RiRT;
+    wb[4] += rhob * o.iRT;
+}
+
+// Roe flux reverse: wLb, wRb += (dF/dw)^T Fb.  Arithmetic and registers bound
+// the kernels that call it: quotients by one divisor share a reciprocal,
+// h and c^2 come from T, and the reverse runs on normalised quantities, about
+// half the instructions of a reverse of the forward formulas as they stand
+// (interior face adjoint of a 64-cell tile in FP32: 1756 -> 996 vector
+// instructions per wave, 199 -> 100 registers).
+template <typename T>
+ADFVM_HD void roe_flux_vjp(const Phys<T>& ph, const T* wL, const T* wR, const T* n, const T* Fb, T* wLb, T* wRb) {
+    const T gm1 = ph.gamma - T(1);
+    RoeSide<T> L, R;
+    RoeFace<T> f;
+    roe_side(ph, wL, n, L);
+    roe_side(ph, wR, n, R);
+    roe_face(ph, wL, L, wR, R, n, f);
+    // F = (central - dissipation)/2: H the adjoint of either half
+    T H[5];
+    for (int i = 0; i < 5; i++) H[i] = T(0.5) * Fb[i];
+    const T Hn = H[1] * n[0] + H[2] * n[1] + H[3] * n[2];
+    // dissipation: l1 drho + s6, l1 drhoU + U s6 - n s7, l1 drhoE + h s6 - Un s7
+    T l1b = -(H[0] * f.drho + H[1] * f.drhoU[0] + H[2] * f.drhoU[1] + H[3] * f.drhoU[2] + H[4] * f.drhoE);
+    const T s6b = -(H[0] + H[1] * f.U[0] + H[2] * f.U[1] + H[3] * f.U[2] + H[4] * f.h);
+    const T s7b = Hn + H[4] * f.Un;
+    T drhob = -H[0] * f.l1, drhoEb = -H[4] * f.l1, hb = -H[4] * f.s6, Unb = H[4] * f.s7;
+    T drhoUb[3], Ub[3];
     for (int i = 0; i < 3; i++) {
-        T b = Fb[1 + i];
-        FU0b[i] = b;
-        l1b += -T(0.5) * b * drhoU[i];
-        drhoUb[i] += -T(0.5) * b * l1;
-        UFb[i] += -T(0.5) * b * abv6;
-        abv6b += -T(0.5) * b * UF[i];
-        abv7b += T(0.5) * b * n[i];
+        drhoUb[i] = -H[1 + i] * f.l1;
+        Ub[i] = -H[1 + i] * f.s6;
     }
-    T FE0b = Fb[4];
-    l1b += -T(0.5) * Fb[4] * drhoE;
-    drhoEb += -T(0.5) * Fb[4] * l1;
-    hFb += -T(0.5) * Fb[4] * abv6;
-    abv6b += -T(0.5) * Fb[4] * hF;
-    UnFb += T(0.5) * Fb[4] * abv7;
-    abv7b += T(0.5) * Fb[4] * UnF;
-    // abv7 = abv3*abv5 - abv2*abv4/aF
-    T abv3b = abv7b * abv5, abv5b = abv7b * abv3;
-    T abv2b = -abv7b * abv4 / aF, abv4b = -abv7b * abv2 / aF;
-    T aFb = abv7b * abv2 * abv4 / (aF * aF);
-    // abv6 = abv3*abv4/a2F - abv2*abv5/aF
-    abv3b += abv6b * abv4 / a2F;
-    abv4b += abv6b * abv3 / a2F;
-    T a2Fb = -abv6b * abv3 * abv4 / (a2F * a2F);
-    abv2b += -abv6b * abv5 / aF;
-    abv5b += -abv6b * abv2 / aF;
-    aFb += abv6b * abv2 * abv5 / (aF * aF);
-    // abv5 = UnF*drho - drhoU.n
-    UnFb += abv5b * drho;
-    drhob += abv5b * UnF;
-    for (int i = 0; i < 3; i++) drhoUb[i] += -abv5b * n[i];
-    // abv4 = gm1*(qF*drho - UF.drhoU + drhoE)
-    T t4 = gm1 * abv4b;
-    T qFb = t4 * drho;
-    drhob += t4 * qF;
+    // s6 = k6 ic, k6 = m3 x - m2 y; s7 = m3 y - m2 x
+    const T k6b = s6b * f.ic;
+    const T m3b = k6b * f.x + s7b * f.y;
+    const T m2b = -(k6b * f.y + s7b * f.x);
+    const T xb = k6b * f.m3 - s7b * f.m2;
+    const T yb = s7b * f.m3 - k6b * f.m2;
+    // x = gm1 (q drho - U.drhoU + drhoE) ic: x's own share of the adjoint of c
+    // is -xb x ic, s6's -s6b s6 ic
+    T cb = -(s6b * f.s6 + xb * f.x) * f.ic;
+    const T t = gm1 * xb * f.ic;
+    T qb = t * f.drho;
+    drhob += t * f.q;
+    drhoEb += t;
+    // y = Un drho - drhoU.n
+    Unb += yb * f.drho;
+    drhob += yb * f.Un;
     for (int i = 0; i < 3; i++) {
-        UFb[i] += -t4 * drhoU[i];
-        drhoUb[i] += -t4 * UF[i];
+        Ub[i] -= t * f.drhoU[i];
+        drhoUb[i] -= t * f.U[i] + yb * n[i];
     }
-    drhoEb += t4;
-    // abv3 = abv1 - l1 ; abv1, abv2
-    T abv1b = abv3b;
-    l1b += -abv3b;
-    T l2b = T(0.5) * abv1b + T(0.5) * abv2b;
-    T l3b = T(0.5) * abv1b - T(0.5) * abv2b;
-    // entropy fix
-    T epsb = 0, lam1b, lam2b, lam3b;
-    if (f1) { lam1b = l1b * T(0.5) * lam1 / eps; epsb += l1b * (T(1) - T(0.25) * lam1 * lam1 / (eps * eps)); } else lam1b = l1b;
-    if (f2) { lam2b = l2b * T(0.5) * lam2 / eps; epsb += l2b * (T(1) - T(0.25) * lam2 * lam2 / (eps * eps)); } else lam2b = l2b;
-    if (f3) { lam3b = l3b * T(0.5) * lam3 / eps; epsb += l3b * (T(1) - T(0.25) * lam3 * lam3 / (eps * eps)); } else lam3b = l3b;
-    // eps = 0.5|ea| + 0.5|eb| (+ small)
-    T eab = T(0.5) * sgn(ea) * epsb, ebb = T(0.5) * sgn(eb_) * epsb;
-    T rhoUnLb = eab / rhoL, rhoUnRb = -eab / rhoR;
-    T rhoLb = -eab * rhoUnL / (rhoL * rhoL), rhoRb = eab * rhoUnR / (rhoR * rhoR);
-    T cLb = ebb, cRb = -ebb;
-    T pLb = cLb * g / (T(2) * cL * rhoL), pRb = cRb * g / (T(2) * cR * rhoR);
-    rhoLb += -cLb * g * pL / (T(2) * cL * rhoL * rhoL);
-    rhoRb += -cRb * g * pR / (T(2) * cR * rhoR * rhoR);
-    // lam
-    T s1 = sgn(UnF), s2 = sgn(UnF + aF), s3 = sgn(UnF - aF);
-    UnFb += lam1b * s1 + lam2b * s2 + lam3b * s3;
-    aFb += lam2b * s2 - lam3b * s3;
-    // drhoE
-    T hRb = drhoEb * rhoR, hLb = -drhoEb * rhoL;
-    rhoRb += drhoEb * hR;
-    rhoLb += -drhoEb * hL;
-    pRb += -drhoEb;
-    pLb += drhoEb;
-    T ULb[3] = {0, 0, 0}, URb[3] = {0, 0, 0};
+    // m2 = (l2 - l3)/2, m3 = (l2 + l3)/2 - l1
+    l1b -= m3b;
+    const T l2b = T(0.5) * (m3b + m2b), l3b = T(0.5) * (m3b - m2b);
+    // entropy fix l = lam^2/(4 eps) + eps below 2 eps
+    T epsb = T(0), lam1b = l1b, lam2b = l2b, lam3b = l3b;
+    if (f.f1) { lam1b = T(0.5) * l1b * f.r1; epsb += l1b - l1b * (T(0.25) * f.r1 * f.r1); }
+    if (f.f2) { lam2b = T(0.5) * l2b * f.r2; epsb += l2b - l2b * (T(0.25) * f.r2 * f.r2); }
+    if (f.f3) { lam3b = T(0.5) * l3b * f.r3; epsb += l3b - l3b * (T(0.25) * f.r3 * f.r3); }
+    const T eUn = T(0.5) * sgn(L.Ue - R.Ue) * epsb, ec = T(0.5) * sgn(L.c - R.c) * epsb;
+    const T g1 = lam1b * sgn(f.Un), g2 = lam2b * sgn(f.Un + f.c), g3 = lam3b * sgn(f.Un - f.c);
+    Unb += g1 + g2 + g3;
+    cb += g2 - g3;
+    // c^2 = gm1 (h - q), q = |U|^2/2
+    const T c2b = gm1 * T(0.5) * cb * f.ic;
+    hb += c2b;
+    qb -= c2b;
+    for (int i = 0; i < 3; i++) Ub[i] += Unb * n[i] + qb * f.U[i];
+    // averages: a = sL/(sL + sR) = 1 - b
+    T D = hb * (L.h - R.h);
+    for (int i = 0; i < 3; i++) D += Ub[i] * (wL[i] - wR[i]);
+    D = T(0.5) * D * f.idv;
+    const T mL = L.rho * L.Un, mR = R.rho * R.Un;
+    const T mLb = H[0] + H[1] * wL[0] + H[2] * wL[1] + H[3] * wL[2] + H[4] * L.h;
+    const T mRb = H[0] + H[1] * wR[0] + H[2] * wR[1] + H[3] * wR[2] + H[4] * R.h;
+    const T rhoLb = D * f.b * recip(L.s) - (drhob + drhoUb[0] * wL[0] + drhoUb[1] * wL[1] + drhoUb[2] * wL[2] +
+                                            drhoEb * L.h) + mLb * L.Un;
+    const T rhoRb = (drhob + drhoUb[0] * wR[0] + drhoUb[1] * wR[1] + drhoUb[2] * wR[2] + drhoEb * R.h) -
+                    D * f.a * recip(R.s) + mRb * R.Un;
     for (int i = 0; i < 3; i++) {
-        rhoRb += drhoUb[i] * UR[i];
-        URb[i] += drhoUb[i] * rhoR;
-        rhoLb += -drhoUb[i] * UL[i];
-        ULb[i] += -drhoUb[i] * rhoL;
+        wLb[i] += Ub[i] * f.a - drhoUb[i] * L.rho + H[1 + i] * mL;
+        wRb[i] += Ub[i] * f.b + drhoUb[i] * R.rho + H[1 + i] * mR;
     }
-    rhoRb += drhob;
-    rhoLb += -drhob;
-    for (int i = 0; i < 3; i++) UFb[i] += UnFb * n[i];
-    a2Fb += aFb * T(0.5) / aF;
-    hFb += gm1 * a2Fb;
-    qFb += -gm1 * a2Fb;
-    for (int i = 0; i < 3; i++) UFb[i] += qFb * UF[i];
-    hLb += hFb * sL / dv;
-    hRb += hFb * sR / dv;
-    T sLb = hFb * hL / dv, sRb = hFb * hR / dv;
-    T dvb = -hFb * hF / dv;
-    for (int i = 0; i < 3; i++) {
-        ULb[i] += UFb[i] * sL / dv;
-        URb[i] += UFb[i] * sR / dv;
-        sLb += UFb[i] * UL[i] / dv;
-        sRb += UFb[i] * UR[i] / dv;
-        dvb += -UFb[i] * UF[i] / dv;
-    }
-    sLb += dvb;
-    sRb += dvb;
-    rhoLb += sLb * T(0.5) / sL;
-    rhoRb += sRb * T(0.5) / sR;
-    // FE0 = 0.5*(rhoUnL*hL + rhoUnR*hR)
-    rhoUnLb += T(0.5) * FE0b * hL;
-    hLb += T(0.5) * FE0b * rhoUnL;
-    rhoUnRb += T(0.5) * FE0b * hR;
-    hRb += T(0.5) * FE0b * rhoUnR;
-    // FU0
-    for (int i = 0; i < 3; i++) {
-        rhoUnLb += T(0.5) * FU0b[i] * UL[i];
-        ULb[i] += T(0.5) * FU0b[i] * rhoUnL;
-        rhoUnRb += T(0.5) * FU0b[i] * UR[i];
-        URb[i] += T(0.5) * FU0b[i] * rhoUnR;
-        pLb += T(0.5) * FU0b[i] * n[i];
-        pRb += T(0.5) * FU0b[i] * n[i];
-    }
-    rhoUnLb += T(0.5) * Fr0b;
-    rhoUnRb += T(0.5) * Fr0b;
-    // h = g p/(gm1 rho) + 0.5 U.U
-    pLb += hLb * g / (gm1 * rhoL);
-    rhoLb += -hLb * g * pL / (gm1 * rhoL * rhoL);
-    pRb += hRb * g / (gm1 * rhoR);
-    rhoRb += -hRb * g * pR / (gm1 * rhoR * rhoR);
-    for (int i = 0; i < 3; i++) { ULb[i] += hLb * UL[i]; URb[i] += hRb * UR[i]; }
-    // rhoUn = rho*Un
-    rhoLb += rhoUnLb * UnL;
-    rhoRb += rhoUnRb * UnR;
-    T UnLb = rhoUnLb * rhoL, UnRb = rhoUnRb * rhoR;
-    for (int i = 0; i < 3; i++) { ULb[i] += UnLb * n[i]; URb[i] += UnRb * n[i]; }
-    for (int i = 0; i < 3; i++) { wLb[i] += ULb[i]; wRb[i] += URb[i]; }
-    wLb[4] += pLb; wRb[4] += pRb;
-    qLb[0] += rhoLb; qRb[0] += rhoRb;
+    wLb[4] += Hn + drhoEb;
+    wRb[4] += Hn - drhoEb;
+    roe_side_vjp(ph, wL, n, L, mLb * L.rho + eUn, rhoLb, hb * f.a - drhoEb * L.rho + H[4] * mL, ec, wLb);
+    roe_side_vjp(ph, wR, n, R, mRb * R.rho - eUn, rhoRb, hb * f.b + drhoEb * R.rho + H[4] * mR, -ec, wRb);
 }
 
 // Lax-Friedrichs flux reverse.  Inputs used: U, p (w) and rho, rhoU, rhoE (q).
@@ -319,74 +328,66 @@ template <typename T>
 ADFVM_HD void viscous_flux_vjp(const Phys<T>& ph, T TL, T TR, const T* UL, const T* UR, T TF, const T* UF,
                                const T* gTF0, const T* gUF0, const T* n, T delta, const T* D, const T* Fb,
                                T* TLb, T* TRb, T* ULb, T* URb, T* TFb, T* UFb, T* gTF0b, T* gUF0b) {
-    T mu = viscosity(ph, TF);
-    T kappa = mu * (ph.Cp / ph.Pr);
-    T snT = (TR - TL) / delta;
-    T gTD = gTF0[0] * D[0] + gTF0[1] * D[1] + gTF0[2] * D[2];
-    T gT[3];
-    for (int k = 0; k < 3; k++) gT[k] = gTF0[k] + snT * D[k] - gTD * D[k];
+    const T mu = viscosity(ph, TF);
+    const T kappa = mu * (ph.Cp / ph.Pr);
+    const T id = recip(delta);
     T gU[9];
     for (int i = 0; i < 3; i++) {
-        T snU = (UR[i] - UL[i]) / delta;
-        T gD = gUF0[3 * i] * D[0] + gUF0[3 * i + 1] * D[1] + gUF0[3 * i + 2] * D[2];
-        for (int k = 0; k < 3; k++) gU[3 * i + k] = gUF0[3 * i + k] + snU * D[k] - gD * D[k];
+        T c = (UR[i] - UL[i]) * id - (gUF0[3 * i] * D[0] + gUF0[3 * i + 1] * D[1] + gUF0[3 * i + 2] * D[2]);
+        for (int k = 0; k < 3; k++) gU[3 * i + k] = gUF0[3 * i + k] + c * D[k];
     }
-    T gTn = gT[0] * n[0] + gT[1] * n[1] + gT[2] * n[2];
-    T tmp3 = gU[0] + gU[4] + gU[8];
-    T t2[3], sigma[3];
+    const T tr = T(2.0 / 3.0) * (gU[0] + gU[4] + gU[8]);
+    T t2[3];                                     // sigma = mu t2
+    for (int i = 0; i < 3; i++)
+        t2[i] = (gU[3 * i] + gU[i]) * n[0] + (gU[3 * i + 1] + gU[3 + i]) * n[1] + (gU[3 * i + 2] + gU[6 + i]) * n[2] -
+                tr * n[i];
+    // reverse: F[1+i] -= sigma_i, F[4] -= q + sigma.UF
+    T sb[3];                                     // adjoint of sigma
     for (int i = 0; i < 3; i++) {
-        t2[i] = (gU[3 * i] + gU[i]) * n[0] + (gU[3 * i + 1] + gU[3 + i]) * n[1] + (gU[3 * i + 2] + gU[6 + i]) * n[2];
-        sigma[i] = mu * (t2[i] - T(2.0 / 3.0) * tmp3 * n[i]);
+        sb[i] = -Fb[1 + i] - Fb[4] * UF[i];
+        UFb[i] -= Fb[4] * (mu * t2[i]);
     }
-    // reverse
-    T sigb[3];
-    for (int i = 0; i < 3; i++) {
-        sigb[i] = -Fb[1 + i] - Fb[4] * UF[i];
-        UFb[i] += -Fb[4] * sigma[i];
+    const T qFb = -Fb[4];
+    if (ph.muModel != 0) {                       // the viscosity's own adjoint, into TF
+        T cT = (TR - TL) * id - (gTF0[0] * D[0] + gTF0[1] * D[1] + gTF0[2] * D[2]);
+        T gTn = T(0);
+        for (int k = 0; k < 3; k++) gTn += (gTF0[k] + cT * D[k]) * n[k];
+        const T mub = sb[0] * t2[0] + sb[1] * t2[1] + sb[2] * t2[2] + qFb * gTn * (ph.Cp / ph.Pr);
+        *TFb += mub * viscosity_dT(ph, TF);
     }
-    T qFb = -Fb[4];
-    T mub = 0, tmp3b = 0, t2b[3];
-    for (int i = 0; i < 3; i++) {
-        mub += sigb[i] * (t2[i] - T(2.0 / 3.0) * tmp3 * n[i]);
-        t2b[i] = sigb[i] * mu;
-        tmp3b += -T(2.0 / 3.0) * sigb[i] * mu * n[i];
-    }
-    T gUb[9];
+    // t2 = (gU + gU^T) n - 2/3 tr(gU) n: a symmetric adjoint B of gU, of
+    // which the part along D goes to the difference across the face
+    for (int i = 0; i < 3; i++) sb[i] *= mu;
+    const T trb = -T(2.0 / 3.0) * (sb[0] * n[0] + sb[1] * n[1] + sb[2] * n[2]);
+    T B[9];
     for (int a = 0; a < 3; a++)
-        for (int b = 0; b < 3; b++) gUb[3 * a + b] = t2b[a] * n[b] + t2b[b] * n[a];
-    gUb[0] += tmp3b; gUb[4] += tmp3b; gUb[8] += tmp3b;
-    T kappab = qFb * gTn;
-    T gTb[3];
-    for (int k = 0; k < 3; k++) gTb[k] = qFb * kappa * n[k];
+        for (int b = a; b < 3; b++) B[3 * a + b] = B[3 * b + a] = sb[a] * n[b] + sb[b] * n[a] + (a == b ? trb : T(0));
     for (int i = 0; i < 3; i++) {
-        T snUb = 0, gDb = 0;
-        for (int k = 0; k < 3; k++) {
-            gUF0b[3 * i + k] += gUb[3 * i + k];
-            snUb += gUb[3 * i + k] * D[k];
-            gDb += -gUb[3 * i + k] * D[k];
-        }
-        for (int k = 0; k < 3; k++) gUF0b[3 * i + k] += gDb * D[k];
-        URb[i] += snUb / delta;
-        ULb[i] += -snUb / delta;
+        const T along = B[3 * i] * D[0] + B[3 * i + 1] * D[1] + B[3 * i + 2] * D[2];
+        for (int k = 0; k < 3; k++) gUF0b[3 * i + k] += B[3 * i + k] - along * D[k];
+        URb[i] += along * id;
+        ULb[i] -= along * id;
     }
-    T snTb = 0, gTDb = 0;
-    for (int k = 0; k < 3; k++) {
-        gTF0b[k] += gTb[k];
-        snTb += gTb[k] * D[k];
-        gTDb += -gTb[k] * D[k];
-    }
-    for (int k = 0; k < 3; k++) gTF0b[k] += gTDb * D[k];
-    *TRb += snTb / delta;
-    *TLb += -snTb / delta;
-    mub += kappab * (ph.Cp / ph.Pr);
-    *TFb += mub * viscosity_dT(ph, TF);
+    const T z = qFb * kappa;
+    const T along = z * (n[0] * D[0] + n[1] * D[1] + n[2] * D[2]);
+    for (int k = 0; k < 3; k++) gTF0b[k] += z * n[k] - along * D[k];
+    *TRb += along * id;
+    *TLb -= along * id;
 }
 
 template <typename T>
-ADFVM_HD void riemann_vjp(const Phys<T>& ph, int which, const T* wL, const T* qL, const T* wR, const T* qR,
-                          const T* n, const T* Fb, T* wLb, T* qLb, T* wRb, T* qRb) {
-    if (which == 0) roe_flux_vjp(ph, wL, qL, wR, qR, n, Fb, wLb, qLb, wRb, qRb);
-    else lf_flux_vjp(ph, wL, qL, wR, qR, n, Fb, wLb, qLb, wRb, qRb);
+ADFVM_HD void riemann_vjp(const Phys<T>& ph, int which, const T* wL, const T* wR, const T* n, const T* Fb, T* wLb,
+                          T* wRb) {
+    if (which == 0) {
+        roe_flux_vjp(ph, wL, wR, n, Fb, wLb, wRb);
+    } else {
+        T qL[5], qR[5], qLb[5] = {0, 0, 0, 0, 0}, qRb[5] = {0, 0, 0, 0, 0};
+        conservative(ph, wL, qL);
+        conservative(ph, wR, qR);
+        lf_flux_vjp(ph, wL, qL, wR, qR, n, Fb, wLb, qLb, wRb, qRb);
+        conservative_vjp(ph, wL, qLb, wLb);
+        conservative_vjp(ph, wR, qRb, wRb);
+    }
 }
 
 // Reverse of face_flux with respect to the F output (the lam output's
@@ -396,7 +397,8 @@ template <typename T>
 ADFVM_HD void face_flux_vjp(const Phys<T>& ph, int kind, const T* wP, const T* gP, const T* wN, const T* gN,
                             const FaceGeo<T>& f, const T* Fb, T* wPb, T* gPb, T* wNb, T* gNb) {
     T TF, UF[3], gTF[3], gUF[9];
-    T wLF[5], qLF[5], wRF[5], qRF[5];
+    T wLF[5], wRF[5];
+    int takenL = 0, takenR = 0;
     if (kind == FACE_BOUNDARY) {
         TF = wN[3];
         for (int i = 0; i < 3; i++) UF[i] = wN[i];
@@ -404,7 +406,7 @@ ADFVM_HD void face_flux_vjp(const Phys<T>& ph, int kind, const T* wP, const T* g
         for (int k = 0; k < 9; k++) gUF[k] = gN[k];
     } else {
         reconstruct(wP, gP, wN, f.lw0, f.qw0, wLF, ph.limit);
-        conservative(ph, wLF, qLF);
+        if (ph.limit) takenL = reconstruct_taken(wP, gP, wN, f.lw0, f.qw0);
         if (kind == FACE_CHARACTERISTIC) {
             for (int i = 0; i < 5; i++) wRF[i] = wN[i];
             TF = wN[3];
@@ -413,12 +415,12 @@ ADFVM_HD void face_flux_vjp(const Phys<T>& ph, int kind, const T* wP, const T* g
             for (int k = 0; k < 9; k++) gUF[k] = gN[k];
         } else {
             reconstruct(wN, gN, wP, f.lw1, f.qw1, wRF, ph.limit);
+            if (ph.limit) takenR = reconstruct_taken(wN, gN, wP, f.lw1, f.qw1);
             for (int i = 0; i < 3; i++) UF[i] = T(0.5) * (wLF[i] + wRF[i]);
             TF = T(0.5) * (wLF[3] + wRF[3]);
             for (int k = 0; k < 3; k++) gTF[k] = T(0.5) * (gP[9 + k] + gN[9 + k]);
             for (int k = 0; k < 9; k++) gUF[k] = T(0.5) * (gP[k] + gN[k]);
         }
-        conservative(ph, wRF, qRF);
     }
     // viscous part
     T TFb = 0, UFb[3] = {0, 0, 0}, gTFb[3] = {0, 0, 0}, gUFb[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
@@ -447,27 +449,24 @@ ADFVM_HD void face_flux_vjp(const Phys<T>& ph, int kind, const T* wP, const T* g
         return;
     }
     T wLFb[5] = {0, 0, 0, 0, 0}, wRFb[5] = {0, 0, 0, 0, 0};
-    T qLFb[5] = {0, 0, 0, 0, 0}, qRFb[5] = {0, 0, 0, 0, 0};
     if (kind == FACE_CHARACTERISTIC) {
         wNb[3] += TFb;
         for (int i = 0; i < 3; i++) wNb[i] += UFb[i];
         for (int k = 0; k < 3; k++) gNb[9 + k] += gTFb[k];
         for (int k = 0; k < 9; k++) gNb[k] += gUFb[k];
-        riemann_vjp(ph, ph.boundaryRiemann, wLF, qLF, wRF, qRF, f.n, Fb, wLFb, qLFb, wRFb, qRFb);
+        riemann_vjp(ph, ph.boundaryRiemann, wLF, wRF, f.n, Fb, wLFb, wRFb);
     } else {
         for (int i = 0; i < 3; i++) { wLFb[i] += T(0.5) * UFb[i]; wRFb[i] += T(0.5) * UFb[i]; }
         wLFb[3] += T(0.5) * TFb; wRFb[3] += T(0.5) * TFb;
         for (int k = 0; k < 3; k++) { gPb[9 + k] += T(0.5) * gTFb[k]; gNb[9 + k] += T(0.5) * gTFb[k]; }
         for (int k = 0; k < 9; k++) { gPb[k] += T(0.5) * gUFb[k]; gNb[k] += T(0.5) * gUFb[k]; }
-        riemann_vjp(ph, ph.riemann, wLF, qLF, wRF, qRF, f.n, Fb, wLFb, qLFb, wRFb, qRFb);
+        riemann_vjp(ph, ph.riemann, wLF, wRF, f.n, Fb, wLFb, wRFb);
     }
-    conservative_vjp(ph, wLF, qLFb, wLFb);
-    conservative_vjp(ph, wRF, qRFb, wRFb);
-    reconstruct_vjp(wP, gP, wN, f.lw0, f.qw0, wLFb, ph.limit, wPb, gPb, wNb);
+    reconstruct_vjp(f.lw0, f.qw0, wLFb, takenL, wPb, gPb, wNb);
     if (kind == FACE_CHARACTERISTIC) {
         for (int i = 0; i < 5; i++) wNb[i] += wRFb[i];
     } else {
-        reconstruct_vjp(wN, gN, wP, f.lw1, f.qw1, wRFb, ph.limit, wNb, gNb, wPb);
+        reconstruct_vjp(f.lw1, f.qw1, wRFb, takenR, wNb, gNb, wPb);
     }
 }
 

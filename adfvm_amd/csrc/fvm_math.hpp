@@ -17,7 +17,33 @@
 namespace adfvm {
 
 template <typename T> ADFVM_HD T fsqrt(T x) { return sqrt(x); }
+template <typename T> ADFVM_HD T recip(T x) { return T(1) / x; }
+// FP32 on the device: the hardware square root and reciprocal (1 ulp each).
+// A quotient compiles to the same reciprocal and product between two exponent
+// scalings (8 instructions) that only matter for divisors below 1.2e-38 or
+// above 8.5e37; the divisors here (densities, temperatures, sound speeds,
+// cell distances and volumes, an eigenvalue floor of at least Phys::small)
+// lie within, and a zero or infinite one gives what the quotient gives.
+#if defined(__HIP_DEVICE_COMPILE__)
+ADFVM_HD float fsqrt(float x) { return __builtin_amdgcn_sqrtf(x); }
+ADFVM_HD float recip(float x) { return __builtin_amdgcn_rcpf(x); }
+#endif
+// Quotients by one divisor.  FP32 shares the reciprocal and has the bits of
+// the quotients (the product is rounded before anything is added to it, being
+// a function's result); otherwise they are quotients.
+template <typename T> struct Divisor {
+    T y;
+    ADFVM_HD explicit Divisor(T y_) : y(y_) {}
+    ADFVM_HD T operator()(T x) const { return x / y; }
+};
+template <> struct Divisor<float> {
+    float iy;
+    ADFVM_HD explicit Divisor(float y) : iy(recip(y)) {}
+    ADFVM_HD float operator()(float x) const { return x * iy; }
+};
 template <typename T> ADFVM_HD T fabs_(T x) { return x < T(0) ? -x : x; }
+ADFVM_HD float fabs_(float x) { return __builtin_fabsf(x); }     // an operand modifier on the device
+ADFVM_HD double fabs_(double x) { return __builtin_fabs(x); }
 template <typename T> ADFVM_HD T fmax_(T a, T b) { return a > b ? a : b; }
 
 template <typename T>
@@ -39,8 +65,9 @@ template <typename T> ADFVM_HD T viscosity(const Phys<T>& ph, T Tf) {
 // RCF.primitive, adFVM/density.py:162-171
 template <typename T> ADFVM_HD void primitive(const Phys<T>& ph, const T* q, T* w) {
     T rho = q[0];
-    T Ux = q[1] / rho, Uy = q[2] / rho, Uz = q[3] / rho;
-    T E = q[4] / rho;
+    const Divisor<T> over_rho(rho);
+    T Ux = over_rho(q[1]), Uy = over_rho(q[2]), Uz = over_rho(q[3]);
+    T E = over_rho(q[4]);
     T e = E - T(0.5) * (Ux * Ux + Uy * Uy + Uz * Uz);
     w[0] = Ux; w[1] = Uy; w[2] = Uz;
     w[4] = (ph.gamma - T(1)) * rho * e;
@@ -50,7 +77,7 @@ template <typename T> ADFVM_HD void primitive(const Phys<T>& ph, const T* q, T* 
 // RCF.conservative, adFVM/density.py:173-181
 template <typename T> ADFVM_HD void conservative(const Phys<T>& ph, const T* w, T* q) {
     T e = ph.Cv * w[3];
-    T rho = w[4] / (e * (ph.gamma - T(1)));
+    T rho = Divisor<T>(e * (ph.gamma - T(1)))(w[4]);
     T U2 = w[0] * w[0] + w[1] * w[1] + w[2] * w[2];
     q[0] = rho;
     q[4] = rho * (e + T(0.5) * U2);
@@ -86,18 +113,18 @@ ADFVM_HD void roe_flux(const Phys<T>& ph, const T* wL, const T* qL, const T* wR,
     T UnL = UL[0] * n[0] + UL[1] * n[1] + UL[2] * n[2];
     T UnR = UR[0] * n[0] + UR[1] * n[1] + UR[2] * n[2];
     T rhoUnL = rhoL * UnL, rhoUnR = rhoR * UnR;
-    T hL = g * pL / (gm1 * rhoL) + T(0.5) * (UL[0] * UL[0] + UL[1] * UL[1] + UL[2] * UL[2]);
-    T hR = g * pR / (gm1 * rhoR) + T(0.5) * (UR[0] * UR[0] + UR[1] * UR[1] + UR[2] * UR[2]);
+    T hL = Divisor<T>(gm1 * rhoL)(g * pL) + T(0.5) * (UL[0] * UL[0] + UL[1] * UL[1] + UL[2] * UL[2]);
+    T hR = Divisor<T>(gm1 * rhoR)(g * pR) + T(0.5) * (UR[0] * UR[0] + UR[1] * UR[1] + UR[2] * UR[2]);
     T Fr = T(0.5) * (rhoUnL + rhoUnR);
     T FU[3];
     for (int i = 0; i < 3; i++) FU[i] = T(0.5) * (rhoUnL * UL[i] + rhoUnR * UR[i] + (pL + pR) * n[i]);
     T FE = T(0.5) * (rhoUnL * hL + rhoUnR * hR);
 
     T sL = fsqrt(rhoL), sR = fsqrt(rhoR);
-    T dv = sL + sR;
+    const Divisor<T> over_s(sL + sR);
     T UF[3];
-    for (int i = 0; i < 3; i++) UF[i] = (UL[i] * sL + UR[i] * sR) / dv;
-    T hF = (hL * sL + hR * sR) / dv;
+    for (int i = 0; i < 3; i++) UF[i] = over_s(UL[i] * sL + UR[i] * sR);
+    T hF = over_s(hL * sL + hR * sR);
     T qF = T(0.5) * (UF[0] * UF[0] + UF[1] * UF[1] + UF[2] * UF[2]);
     T a2F = gm1 * (hF - qF);
     T aF = fsqrt(a2F);
@@ -109,20 +136,22 @@ ADFVM_HD void roe_flux(const Phys<T>& ph, const T* wL, const T* qL, const T* wR,
     T drhoE = (hR * rhoR - pR) - (hL * rhoL - pL);
 
     T lam1 = fabs_(UnF), lam2 = fabs_(UnF + aF), lam3 = fabs_(UnF - aF);
-    T eps = T(0.5) * fabs_(rhoUnL / rhoL - rhoUnR / rhoR);
-    eps += T(0.5) * fabs_(fsqrt(g * pL / rhoL) - fsqrt(g * pR / rhoR));
-    eps = eps < T(0) ? eps - ph.small : eps + ph.small;
+    const Divisor<T> over_rhoL(rhoL), over_rhoR(rhoR);
+    T eps = T(0.5) * fabs_(over_rhoL(rhoUnL) - over_rhoR(rhoUnR));
+    eps += T(0.5) * fabs_(fsqrt(over_rhoL(g * pL)) - fsqrt(over_rhoR(g * pR)));
+    eps = eps + ph.small;
     T e2 = T(2) * eps;
-    if (lam1 < e2) lam1 = T(0.25) * lam1 * lam1 / eps + eps;
-    if (lam2 < e2) lam2 = T(0.25) * lam2 * lam2 / eps + eps;
-    if (lam3 < e2) lam3 = T(0.25) * lam3 * lam3 / eps + eps;
+    const Divisor<T> over_eps(eps);
+    if (lam1 < e2) lam1 = over_eps(T(0.25) * lam1 * lam1) + eps;
+    if (lam2 < e2) lam2 = over_eps(T(0.25) * lam2 * lam2) + eps;
+    if (lam3 < e2) lam3 = over_eps(T(0.25) * lam3 * lam3) + eps;
 
     T abv1 = T(0.5) * (lam2 + lam3);
     T abv2 = T(0.5) * (lam2 - lam3);
     T abv3 = abv1 - lam1;
     T abv4 = gm1 * (qF * drho - (UF[0] * drhoU[0] + UF[1] * drhoU[1] + UF[2] * drhoU[2]) + drhoE);
     T abv5 = UnF * drho - (drhoU[0] * n[0] + drhoU[1] * n[1] + drhoU[2] * n[2]);
-    T abv6 = abv3 * abv4 / a2F - abv2 * abv5 / aF;
+    T abv6 = Divisor<T>(a2F)(abv3 * abv4) - Divisor<T>(aF)(abv2 * abv5);
     T abv7 = abv3 * abv5 - abv2 * abv4 / aF;
 
     F[0] = Fr - T(0.5) * (lam1 * drho + abv6);
@@ -156,13 +185,14 @@ ADFVM_HD void viscous_flux(const Phys<T>& ph, T TL, T TR, const T* UL, const T* 
                            const T* D, T* F) {
     T mu = viscosity(ph, TF);
     T kappa = mu * (ph.Cp / ph.Pr);
-    T snT = (TR - TL) / delta;
+    const Divisor<T> over_delta(delta);
+    T snT = over_delta(TR - TL);
     T gTD = gTF0[0] * D[0] + gTF0[1] * D[1] + gTF0[2] * D[2];
     T gT[3];
     for (int k = 0; k < 3; k++) gT[k] = gTF0[k] + snT * D[k] - gTD * D[k];
     T gU[9];
     for (int i = 0; i < 3; i++) {
-        T snU = (UR[i] - UL[i]) / delta;
+        T snU = over_delta(UR[i] - UL[i]);
         T gD = gUF0[3 * i] * D[0] + gUF0[3 * i + 1] * D[1] + gUF0[3 * i + 2] * D[2];
         for (int k = 0; k < 3; k++) gU[3 * i + k] = gUF0[3 * i + k] + snU * D[k] - gD * D[k];
     }
