@@ -529,8 +529,9 @@ class Context(object):
         return out
 
     def autotune(self, u, reps=5, stream=None):
-        """Pick each stencil kernel's block size by timing it on state u;
-        returns {kernel: (block, ms per launch)}."""
+        """Time each stencil kernel on state u; returns {kernel: (block, ms
+        per launch)}.  The kernels' cell tiles fix their blocks, so there is
+        nothing to choose."""
         self._check(u, (5, self.nIC))
         self._chk(self.lib.adfvm_autotune(self.handle, _dptr(u), int(reps), _stream(stream)))
         return self.kernel_config()

@@ -43,6 +43,22 @@ template <typename T> ADFVM_HD void primitive_vjp(const Phys<T>& ph, const T* q,
     qb[0] += T(0.5) * gm1 * U2 * pb + (T(0.5) * U2 - e) * Tb / rho - UwU / rho;
 }
 
+// The same at a state given by its primitive values w (e = Cv T,
+// rho = p/((g-1) e)).
+template <typename T> ADFVM_HD void primitive_vjp_at(const Phys<T>& ph, const T* w, const T* wb, T* qb) {
+    const T gm1 = ph.gamma - T(1);
+    const T e = ph.Cv * w[3];
+    const T rho = w[4] / (gm1 * e);
+    const T U2 = w[0] * w[0] + w[1] * w[1] + w[2] * w[2];
+    const T Tb = wb[3] * ph.invCv;
+    const T pb = wb[4];
+    const T eb = Tb / rho + pb * gm1;
+    qb[4] += eb;
+    for (int i = 0; i < 3; i++) qb[1 + i] += wb[i] / rho - eb * w[i];
+    const T UwU = w[0] * wb[0] + w[1] * wb[1] + w[2] * wb[2];
+    qb[0] += T(0.5) * gm1 * U2 * pb + (T(0.5) * U2 - e) * Tb / rho - UwU / rho;
+}
+
 // conservative(w) -> q ; wb += (dq/dw)^T qb
 template <typename T> ADFVM_HD void conservative_vjp(const Phys<T>& ph, const T* w, const T* qb, T* wb) {
     T gm1 = ph.gamma - T(1);

@@ -1,12 +1,12 @@
 // libadfvm: HIP kernels for gfx950 (MI355X) and the C ABI of include/adfvm.h.
 //
 // Design (one GPU, one context per mesh):
-//  * state and gradients are structure-of-arrays rows of nInternalCells
-//    scalars in the context precision (float or double);
-//  * every face->cell accumulation is a gather: each cell walks its six
-//    cellFaces slots in order (owned faces in face order, then neighbour
-//    faces, cmesh.cpp:9-19) and reads what the face kernel stored for them.
-//    No atomics: results are bit-identical from run to run;
+//  * the caller's state and gradient arrays are structure-of-arrays rows of
+//    nInternalCells scalars in the context precision (float or double); the
+//    library's own are records in tile order (tile_kernels.inc);
+//  * every face->cell accumulation is a sum over the cell's six cellFaces
+//    slots in order (owned faces in face order, then neighbour faces,
+//    cmesh.cpp:9-19).  No atomics: results are bit-identical from run to run;
 //  * cyclic ghosts are resolved at set-up to the paired internal cell; the
 //    ghost of a non-cyclic boundary face is evaluated where it is used, from
 //    its owner cell and the patch's values (a ghost array is filled only for
@@ -27,6 +27,7 @@
 #include "fvm_math.hpp"
 #include "adjoint_math.hpp"
 #include "dual.hpp"
+#include "tiles.hpp"
 
 using namespace adfvm;
 
@@ -42,19 +43,6 @@ __device__ __forceinline__ int xcd_block() {
     const unsigned nb = gridDim.x, b = blockIdx.x;
     const unsigned q = nb >> 3, r = nb & 7u, x = b & 7u, k = b >> 3;
     return (int)(x * q + (x < r ? x : r) + k);
-}
-
-// The face kernels read both cells of a face; there a contiguous eighth per
-// XCD measured slower (though it cut their HBM reads by a fifth), while
-// chunks of 16 consecutive blocks per XCD, the chunks dealt round-robin,
-// measured 1-2% faster than the plain order.  Bijection of [0, gridDim.x)
-// (the last partial chunk keeps the plain order).
-__device__ __forceinline__ int xcd_chunk_block() {
-    const unsigned nb = gridDim.x, b = blockIdx.x, C = 16;
-    const unsigned full = nb / (8u * C) * (8u * C);
-    if (b >= full) return (int)b;
-    const unsigned chunk = b / (8u * C), r = b % (8u * C);
-    return (int)(chunk * 8u * C + (r & 7u) * C + (r >> 3));
 }
 
 // ------------------------------------------------------------- tables ----
@@ -90,10 +78,6 @@ template <typename T> struct DMesh {
     int nIC, nIF, nF, nBF;
     const T* geo;           // [G_ROWS][nF]
     const T* vol;           // [nIC]
-    const T* ngeo;          // [6][3][nIC]: per coupled cell slot, the paired face's owner's gradient
-                            // stencil seen from this cell: coef * S*n / V_other (zero elsewhere)
-    const T* sgeo;          // [6][4][nIC]: per cell slot, S*n signed outward for the cell (3) and
-                            // the weight of the other side's value in the face value (op.py:47-58)
     const int* sFace;       // [6][nIC]
     const int* sOther;      // [6][nIC]: internal cell, or -1-b for boundary face b
     const unsigned char* sFlags;  // [6][nIC]
@@ -101,9 +85,6 @@ template <typename T> struct DMesh {
     const int* owner;       // [nF]
     const int* fOther;      // [nF]: neighbour, paired internal cell (cyclic) or -1-b (ghost)
     const unsigned char* fKind;  // [nF]: FACE_INTERIOR / FACE_CHARACTERISTIC / FACE_BOUNDARY
-    const int* posP;        // [nF]: record index (plane*nIC + cell) of the face's owner-side adjoint
-    const int* posN;        // [nF]: record index of its neighbour-side adjoint, -1 if none
-    int ownerSum;           // the face adjoint sums each cell's owned internal faces into plane 0
     const int* bPatch;      // [nBF]
     const DPatch* patches;
     const T* bcval;
@@ -129,17 +110,17 @@ template <bool ST, typename T> __device__ __forceinline__ void st(T* p, T v) {
     else *p = v;
 }
 
-template <bool ST, typename T> __device__ __forceinline__ void load_geo(const DMesh<T>& m, int f, FaceGeo<T>& g) {
-    const T* G = m.geo;
-    const long s = m.nF;
-    g.A = ld<ST>(G + G_A * s + f);
-    g.n[0] = ld<ST>(G + G_NX * s + f); g.n[1] = ld<ST>(G + G_NY * s + f); g.n[2] = ld<ST>(G + G_NZ * s + f);
-    g.w = T(0);           // the face weight enters gradients only (slot geometry), not the face flux
-    g.delta = ld<ST>(G + G_DELTA * s + f);
-    g.D[0] = ld<ST>(G + G_DX * s + f); g.D[1] = ld<ST>(G + G_DY * s + f); g.D[2] = ld<ST>(G + G_DZ * s + f);
-    g.lw0 = ld<ST>(G + G_LW0 * s + f); g.lw1 = ld<ST>(G + G_LW1 * s + f);
-    g.qw0[0] = ld<ST>(G + G_Q0X * s + f); g.qw0[1] = ld<ST>(G + G_Q0Y * s + f); g.qw0[2] = ld<ST>(G + G_Q0Z * s + f);
-    g.qw1[0] = ld<ST>(G + G_Q1X * s + f); g.qw1[1] = ld<ST>(G + G_Q1Y * s + f); g.qw1[2] = ld<ST>(G + G_Q1Z * s + f);
+// Geometry of face f.
+template <typename T> __device__ __forceinline__ void load_geo(const DMesh<T>& m, int f, FaceGeo<T>& g) {
+    auto row = [&](int r) { return m.geo[(long)r * m.nF + f]; };
+    g.A = row(G_A);
+    g.n[0] = row(G_NX); g.n[1] = row(G_NY); g.n[2] = row(G_NZ);
+    g.w = row(G_W);
+    g.delta = row(G_DELTA);
+    g.D[0] = row(G_DX); g.D[1] = row(G_DY); g.D[2] = row(G_DZ);
+    g.lw0 = row(G_LW0); g.lw1 = row(G_LW1);
+    g.qw0[0] = row(G_Q0X); g.qw0[1] = row(G_Q0Y); g.qw0[2] = row(G_Q0Z);
+    g.qw1[0] = row(G_Q1X); g.qw1[1] = row(G_Q1Y); g.qw1[2] = row(G_Q1Z);
 }
 
 // primitive values of a value source: internal cell (from the state) or ghost.
@@ -158,15 +139,8 @@ __device__ __forceinline__ void load_prim(const Phys<T>& ph, const T* __restrict
     for (int i = 0; i < 5; i++) w[i] = internal ? p[i] : q[i];
 }
 
-// Internal work buffers are arrays of records so that a gathered record is a
-// few vector loads instead of one cache line per field:
-//   gradients        [nIC][GREC]   15 used (padded to 16-byte multiples)
-//   face fluxes      [nF][FREC]    F*A (5), lam*A, unpadded: 24 B in FP32 (48 B in
-//                                  FP64), accessed as pairs of scalars
-//   face adjoints    [nPlanes][nIC][AREC] one plane per cell slot, then cyclic
-//                                  extras: gradient adjoint (15), primitive adjoint (5)
-//   cell adjoints    [nIC][AREC]   same layout as one side of a face record
-constexpr int GREC = 16, FREC = 6, AREC = 20;
+// cell adjoint records: gradient adjoint (15), primitive adjoint (5)
+constexpr int AREC = 20;
 
 // N contiguous values from / to a 16-byte aligned address (N a multiple of
 // 16/sizeof(T)), as 16-byte memory operations.  The copies go through
@@ -184,28 +158,6 @@ template <int N, typename T> __device__ __forceinline__ void vstore(T* __restric
     T* a = static_cast<T*>(__builtin_assume_aligned(p, 16));
 #pragma unroll
     for (int k = 0; k < (int)(N * sizeof(T) / 16); k++) __builtin_memcpy(a + k * (16 / sizeof(T)), in + k * (16 / sizeof(T)), 16);
-}
-
-// Records of an even number of scalars aligned to a pair of them (the face
-// flux records): pairs of scalars per access.
-template <int N, typename T> __device__ __forceinline__ void pload(const T* __restrict__ p, T* out) {
-    static_assert(N % 2 == 0, "pairs");
-    const T* a = static_cast<const T*>(__builtin_assume_aligned(p, 2 * sizeof(T)));
-#pragma unroll
-    for (int k = 0; k < N / 2; k++) __builtin_memcpy(out + 2 * k, a + 2 * k, 2 * sizeof(T));
-}
-template <int N, typename T> __device__ __forceinline__ void pstore(T* __restrict__ p, const T* in) {
-    static_assert(N % 2 == 0, "pairs");
-    T* a = static_cast<T*>(__builtin_assume_aligned(p, 2 * sizeof(T)));
-#pragma unroll
-    for (int k = 0; k < N / 2; k++) __builtin_memcpy(a + 2 * k, in + 2 * k, 2 * sizeof(T));
-}
-
-// the 15 gradient entries of cell c (g has room for GREC values)
-template <typename T>
-__device__ __forceinline__ void load_grad(const T* __restrict__ grad, long nIC, int c, T* g) {
-    (void)nIC;
-    vload<GREC>(grad + (long)GREC * c, g);
 }
 
 // ------------------------------------------------------------- kernels ---
@@ -282,59 +234,6 @@ __global__ void __launch_bounds__(BLOCK) ghost_kernel(DMesh<T> m, Phys<T> ph, co
     for (int i = 0; i < 5; i++) ghost[i * nBF + b] = out[i];
 }
 
-// Gauss cell gradients of U, T, p (op.gradCell, op.py:45-63).
-template <typename T, int BS, bool ST, bool GH>
-__global__ void __launch_bounds__(BS) grad_kernel(DMesh<T> m, Phys<T> ph, const T* __restrict__ u,
-                                                     const T* __restrict__ ghost, T* __restrict__ grad) {
-    int c = xcd_block() * BS + threadIdx.x;
-    if (c >= m.nIC) return;
-    const long nIC = m.nIC;
-    const T V = m.vol[c];       // loaded first: read after the slot loop it was a last, unhidden wait
-    T wc[5];
-    load_prim(ph, u, nIC, ghost, m.nBF, c, wc);
-    T g[15];
-    for (int i = 0; i < 15; i++) g[i] = T(0);
-    for (int j = 0; j < 6; j++) {
-        const int o = ld<ST>(m.sOther + j * nIC + c);
-        T wo[5];
-        if constexpr (GH) {
-            // a ghost slot's value from this cell (the face's owner): a copy
-            // without reading the patch when the slot is flagged so
-            const bool copy = ld<ST>(m.sFlags + j * nIC + c) & SLOT_GHOST_COPY;
-            T wi[5], wg[5];
-            load_prim(ph, u, nIC, u, nIC, o < 0 ? c : o, wi);
-            for (int i = 0; i < 5; i++) wg[i] = wc[i];
-            if (o < 0 && !copy) ghost_value(m, ph, -1 - o, wc, wg);
-            for (int i = 0; i < 5; i++) wo[i] = o < 0 ? wg[i] : wi[i];
-        } else {
-            load_prim(ph, u, nIC, ghost, m.nBF, o, wo);
-        }
-        const T* sg = m.sgeo + (long)(4 * j) * nIC + c;
-        const T SN[3] = {ld<ST>(sg), ld<ST>(sg + nIC), ld<ST>(sg + 2 * nIC)};
-        const T w = ld<ST>(sg + 3 * nIC);
-        for (int i = 0; i < 5; i++) {
-            T phiF = wc[i] * (T(1) - w) + wo[i] * w;
-            g[3 * i + 0] += phiF * SN[0];
-            g[3 * i + 1] += phiF * SN[1];
-            g[3 * i + 2] += phiF * SN[2];
-        }
-    }
-    T out[GREC];
-    for (int i = 0; i < 15; i++) out[i] = g[i] / V;
-    out[15] = T(0);
-    vstore<GREC>(grad + (long)GREC * c, out);
-}
-
-// gradient records -> the public [15][nIC] rows
-template <typename T>
-__global__ void __launch_bounds__(BLOCK) grad_rows_kernel(long nIC, const T* __restrict__ grec, T* __restrict__ rows) {
-    long c = (long)blockIdx.x * BLOCK + threadIdx.x;
-    if (c >= nIC) return;
-    T g[GREC];
-    vload<GREC>(grec + GREC * c, g);
-    for (int i = 0; i < 15; i++) rows[i * nIC + c] = g[i];
-}
-
 // Block reduction of one double per thread into out[blockIdx.x]; op 0 sum, 1 max.
 template <int OP, int BS = BLOCK>
 __device__ void block_reduce_store(double v, double* out) {
@@ -372,115 +271,7 @@ __global__ void __launch_bounds__(BLOCK) finalize_kernel(const double* __restric
     if (threadIdx.x == 0) *out = sh[0];
 }
 
-// Face fluxes, one face per thread (faces are in owner order, so the owner
-// reads of neighbouring threads coincide and the geometry rows stream):
-//   fbuf[i][f] = F_i(f)*A_f (i < 5),  fbuf[5][f] = lam_f*A_f
-// Internal and coupled faces: RCF.flux (density.py:253-305) between the
-// owner and the neighbour (for a cyclic face, the paired internal cell);
-// characteristic / other boundary faces: the ghost as the right state.
-template <typename T, int BS, bool ST, bool GH>
-__global__ void __launch_bounds__(BS) face_flux_kernel(DMesh<T> m, Phys<T> ph, const T* __restrict__ u,
-                                                          const T* __restrict__ grad, const T* __restrict__ ghost,
-                                                          T* __restrict__ fbuf) {
-    const int f = xcd_chunk_block() * BS + threadIdx.x;
-    if (f >= m.nF) return;
-    const long nIC = m.nIC, nBF = m.nBF, nF = m.nF;
-    const int P = m.owner[f];
-    const int o = ld<ST>(m.fOther + f);
-    const int kindByte = ld<ST>(m.fKind + f);
-    const int kind = face_kind(kindByte);
-    FaceGeo<T> fg;
-    load_geo<ST>(m, f, fg);
-    T wP[5], gP[GREC], wN[5], gN[GREC], F[5], lam;
-    load_prim(ph, u, nIC, ghost, nBF, P, wP);
-    load_grad(grad, nIC, P, gP);
-    if constexpr (GH) {
-        // a boundary face's ghost from its owner (a copy without reading the
-        // patch when the face is flagged so)
-        T wi[5], wg[5];
-        load_prim(ph, u, nIC, u, nIC, o < 0 ? P : o, wi);
-        for (int i = 0; i < 5; i++) wg[i] = wP[i];
-        if (o < 0 && !(kindByte & FACE_GHOST_COPY)) ghost_value(m, ph, -1 - o, wP, wg);
-        for (int i = 0; i < 5; i++) wN[i] = o < 0 ? wg[i] : wi[i];
-    } else {
-        load_prim(ph, u, nIC, ghost, nBF, o, wN);
-    }
-    if (kind == FACE_INTERIOR) {
-        load_grad(grad, nIC, o, gN);
-        face_flux(ph, FACE_INTERIOR, wP, gP, wN, gN, fg, F, &lam);
-    } else {
-        face_flux(ph, kind, wP, gP, wN, gP, fg, F, &lam);
-    }
-    T rec[FREC];
-    for (int i = 0; i < 5; i++) rec[i] = F[i] * fg.A;
-    rec[5] = lam * fg.A;
-    pstore<FREC>(fbuf + (long)FREC * f, rec);
-    (void)nF;
-}
-
-// Residual and stage update, one cell per thread, gathering the six face
-// fluxes in cellFaces slot order:
-//   L_c = (1/V_c) sum_slots sign*(F A)_f     (op.div, op.py:12-20)
-//   lam_c = (1/V_c) sum_slots (lam A)_f      (op.absDiv, op.py:22-29)
-// MODE 0: uout = a0*u0 + ai*ui + (-beta*(L-S))*dt   (timestep.update, timestep.py:35-45)
-//         with a0 = 1 - ai when u0 is given (every such stage of the tables)
-// MODE 1: uout = L (the residual)
-// The last SSP-RK3 stage passes the step's state as both u0 and uout (each
-// thread reads u0[c] before writing uout[c] at the same index), so neither
-// is declared __restrict__.
-template <typename T, int MODE, int BS, bool ST>
-__global__ void __launch_bounds__(BS) stage_kernel(DMesh<T> m, const T* __restrict__ fbuf,
-                                                      const T* __restrict__ ui, const T* u0,
-                                                      T ai, T nbeta, T dt, const T* __restrict__ S,
-                                                      T* uout, T* __restrict__ dtcCell,
-                                                      double* __restrict__ dtcPartial) {
-    int c = xcd_block() * BS + threadIdx.x;
-    const long nIC = m.nIC, nF = m.nF;
-    double dtcv = 0.0;
-    if (c < m.nIC) {
-        // the cell's own rows first, so their loads overlap the face gathers
-        T v[5], v0[5], sv[5];
-        if (MODE == 0) {
-            for (int i = 0; i < 5; i++) v[i] = ld<ST>(ui + i * nIC + c);
-            for (int i = 0; i < 5; i++) v0[i] = u0 ? ld<ST>(u0 + i * nIC + c) : T(0);
-            for (int i = 0; i < 5; i++) sv[i] = S ? ld<ST>(S + i * nIC + c) : T(0);
-        }
-        T L[5] = {0, 0, 0, 0, 0};
-        T lamSum = 0;
-        for (int j = 0; j < 6; j++) {
-            const int f = ld<ST>(m.sFace + j * nIC + c);
-            const bool own = ld<ST>(m.sFlags + j * nIC + c) & 1;
-            T rec[FREC];
-            pload<FREC>(fbuf + (long)FREC * f, rec);
-            for (int i = 0; i < 5; i++) L[i] += own ? rec[i] : -rec[i];
-            lamSum += rec[5];
-        }
-        (void)nF;
-        const T V = m.vol[c];
-        for (int i = 0; i < 5; i++) L[i] = L[i] / V;
-        lamSum = lamSum / V;
-        if (MODE == 1) {
-            for (int i = 0; i < 5; i++) uout[i * nIC + c] = L[i];
-        } else {
-            for (int i = 0; i < 5; i++) {
-                const T Li = S ? L[i] - sv[i] : L[i];
-                if (u0) {
-                    // a0 = 1 - ai: uout = u0 + (ai*(ui - u0) - beta*(L-S)*dt), the
-                    // change formed at its own scale and added to u0 in one
-                    // rounding.  (ai*ui + a0*u0 rounds ai*ui on a finer grid than
-                    // the sum's; with ai = 2/3 that is biased by -1/9 ulp a step.)
-                    const T du = ai * (v[i] - v0[i]) + (nbeta * Li) * dt;
-                    uout[i * nIC + c] = v0[i] + du;
-                } else {
-                    uout[i * nIC + c] = ai * v[i] + (nbeta * Li) * dt;
-                }
-            }
-        }
-        if (dtcCell) dtcCell[c] = lamSum;
-        dtcv = (double)lamSum;
-    }
-    if (dtcPartial) block_reduce_store<1, BS>(dtcv, dtcPartial);
-}
+#include "tile_kernels.inc"
 
 // Objective partial sums (FP64): kinetic energy 0.5*rho*|U|^2*V per cell.
 template <typename T>
@@ -728,41 +519,31 @@ struct adfvm_ctx {
     int* cellNbFull = nullptr;   // reference cellNeighbours [6][nIC]
     int* nbFull = nullptr;       // ghost-extended neighbour [nF]
     void* ghost = nullptr;
-    void* sgeo = nullptr;      // [6][4][nIC] cell-slot gradient geometry
-    void* ngeo = nullptr;      // [6][3][nIC] cell-slot transposed-stencil coefficients
     void* visc = nullptr;      // adjoint viscosity: [6][nIC] slot coefficients, [nIC] diagonal, [nIC] eigenvalue
-    void* u1 = nullptr; void* u2 = nullptr;
-    void* grad0 = nullptr; void* grad1 = nullptr; void* grad2 = nullptr;
-    void* adjAcc = nullptr;    // [5][nIC] adjoint of u0 accumulated over the stages
-    void* adjG = nullptr;      // [nIC][AREC] cell adjoint records (gradient 15, primitive 5)
+    void* st[3] = {nullptr, nullptr, nullptr};    // state records of the step's start and its intermediate stages
+    void* rows1 = nullptr;     // [5][nIC] the objective stage's state in the caller's numbering
+    void* rec[3] = {nullptr, nullptr, nullptr};   // [nIC][CREC] stage records
+    void* adjU = nullptr;      // [nIC][5] adjoint between the stages
+    void* adjAcc = nullptr;    // [nIC][5] adjoint of u0 accumulated over the stages
+    void* adjG = nullptr;      // [nIC][AREC] cell adjoint records
     double* partial = nullptr; int nPartial = 0;
-    // block size of each tunable stencil kernel (adfvm_autotune) and its measured time
-    int bs[6] = {256, 256, 256, 256, 256, 256};
-    double tuneMs[6] = {-1, -1, -1, -1, -1, -1};
+    double tuneMs[6] = {-1, -1, -1, -1, -1, -1};   // measured time of each stencil kernel (adfvm_autotune)
     // cell segments (adfvm_set_segments): objective per segment
     int nSeg = 1, nSegBlocks = 0;
     long* segCell = nullptr; int* segBlock = nullptr; int* blockSeg = nullptr;
     double* scal = nullptr;    // small device scalars
     int* fOther = nullptr; unsigned char* fKind = nullptr;
-    int* posP = nullptr; int* posN = nullptr;
-    int nPlanes = 6;           // adjoint record planes: one per cell slot, then cyclic extras
-    // internal faces sorted by owner: per block size, the face ranges of the
-    // owner-summing face adjoint blocks (no owner split between two ranges)
-    // boundary faces with a ghost by face kind (0 characteristic, 1 boundary)
-    // boundary faces with a ghost by face kind (characteristic, boundary):
-    // per block of BLOCK threads its first boundary index and face count,
-    // blocks never crossing a gap between runs of one kind
-    int* kindBlk[3] = {nullptr, nullptr, nullptr};
-    int nKindBlk[3] = {0, 0, 0};
-    bool ownerSum = false;
     // the streaming policy (ld / st): non-temporal single-use rows when one
     // stage's working set exceeds the Infinity Cache (adfvm_set_streaming)
     bool stream = false;
-    int* fvjpBlk[4] = {nullptr, nullptr, nullptr, nullptr};
-    int fvjpNBlk[4] = {0, 0, 0, 0};
     void* meshGrad = nullptr;  // caller's mesh-geometry gradient array (adfvm_set_mesh_grad), or none
-    void* fbuf = nullptr;      // [6][nF] face fluxes * area
-    void* frec = nullptr;      // [nPlanes][nIC][AREC] face adjoint records, by cell slot
+    // cell tiles (tiles.hpp), their face geometry and the cell geometry by position
+    int nTiles = 0;
+    long nPos() const { return (long)TILE_CELLS * nTiles; }
+    long nTileFaces() const { return (long)TILE_FACES * nTiles; }
+    int* toUser = nullptr; int* toTile = nullptr; int* tileFaceId = nullptr;
+    unsigned long long* tilePairs = nullptr;
+    unsigned char* tileBlock = nullptr; void* tileFaceW = nullptr;
     // per-kernel event timing (adfvm_profile)
     bool prof = false;
     std::vector<hipEvent_t> evPool;
@@ -813,22 +594,14 @@ int set_err(adfvm_ctx* ctx, int code, const std::string& m) {
 int grid_for(long n) { return (int)((n + BLOCK - 1) / BLOCK); }
 int grid_bs(long n, int bs) { return (int)((n + bs - 1) / bs); }
 
-// Tunable stencil kernels and the block sizes they are built for.
+// The stencil kernels' names and the block sizes adfvm_set_kernel_block
+// takes.  A tile fixes the block at TILE_THREADS (one thread per face of the
+// tile); the flux and the stage update, and the face adjoint and its gather,
+// are one kernel each.
 enum { K_GRAD = 0, K_FLUX, K_STAGE, K_FVJP, K_GATHER, K_GVJP, K_TUNABLE };
 const char* const kTunableName[K_TUNABLE] = {"grad_kernel", "face_flux_kernel", "stage_kernel",
                                               "face_vjp_kernel", "vjp_gather_kernel", "grad_vjp_kernel"};
 const int kBlockChoices[4] = {64, 128, 256, 512};
-int block_choice(int bs) { return bs == 64 ? 0 : bs == 128 ? 1 : bs == 512 ? 3 : 2; }
-
-// Calls f(std::integral_constant<int, BS>) for the block size bs.
-template <typename F> void with_block(int bs, F&& f) {
-    switch (bs) {
-        case 64: f(std::integral_constant<int, 64>()); break;
-        case 128: f(std::integral_constant<int, 128>()); break;
-        case 512: f(std::integral_constant<int, 512>()); break;
-        default: f(std::integral_constant<int, 256>()); break;
-    }
-}
 
 // Calls f(std::bool_constant<st>): the streaming policy of the kernels that
 // take one (ld / st).
@@ -867,13 +640,19 @@ template <typename T> Phys<T> phys_cast(const Phys<double>& p) {
 template <typename T> DMesh<T> dmesh(const adfvm_ctx* c) {
     DMesh<T> m;
     m.nIC = c->nIC; m.nIF = c->nIF; m.nF = c->nF; m.nBF = c->nBF;
-    m.geo = (const T*)c->geo; m.vol = (const T*)c->vol; m.sgeo = (const T*)c->sgeo; m.ngeo = (const T*)c->ngeo;
+    m.geo = (const T*)c->geo; m.vol = (const T*)c->vol; 
     m.sFace = c->sFace; m.sOther = c->sOther; m.sFlags = c->sFlags; m.sPair = c->sPair;
     m.owner = c->owner; m.bPatch = c->bPatch; m.patches = c->patches; m.bcval = (const T*)c->bcval;
     m.fOther = c->fOther; m.fKind = c->fKind;
-    m.posP = c->posP; m.posN = c->posN;
-    m.ownerSum = c->ownerSum ? 1 : 0;
     return m;
+}
+
+template <typename T> DTiles<T> dtiles(const adfvm_ctx* c) {
+    DTiles<T> t;
+    t.n = c->nTiles;
+    t.block = c->tileBlock; t.toUser = c->toUser; t.toTile = c->toTile; t.faceId = c->tileFaceId; t.pairs = c->tilePairs;
+    t.faceW = (const T*)c->tileFaceW;
+    return t;
 }
 
 template <typename T> int upload(adfvm_ctx* ctx, void** dst, const std::vector<T>& v) {
@@ -882,7 +661,8 @@ template <typename T> int upload(adfvm_ctx* ctx, void** dst, const std::vector<T
     return ADFVM_OK;
 }
 
-template <typename T> int create_typed(adfvm_ctx* ctx, const adfvm_solver_desc* d) {
+template <typename T> int create_typed(adfvm_ctx* ctx, const adfvm_solver_desc* d, const Tiles& t) {
+    const std::vector<int>& toUser = t.toUser;
     const long nF = ctx->nF, nIC = ctx->nIC, nBF = ctx->nBF;
     std::vector<T> geo((size_t)G_ROWS * nF);
     for (long f = 0; f < nF; f++) {
@@ -903,43 +683,48 @@ template <typename T> int create_typed(adfvm_ctx* ctx, const adfvm_solver_desc* 
     std::vector<T> vol(nIC);
     for (long c = 0; c < nIC; c++) vol[c] = (T)d->volumes[c];
     if ((rc = upload(ctx, &ctx->vol, vol)) != ADFVM_OK) return rc;
-    // Gauss-gradient geometry per cell slot, computed in FP64 and cast once:
+    const long nPos = ctx->nPos();
+    // Gauss-gradient geometry per cell slot, by position, computed in FP64 and cast once:
     // the cell's outward S*n and the weight w' of the other side's value
     // (phi_f = phi_c (1 - w') + phi_other w'), streamed by the gradient
     // kernels instead of gathering face rows.
-    std::vector<T> sg((size_t)24 * nIC);
-    for (long c = 0; c < nIC; c++)
-        for (int j = 0; j < 6; j++) {
-            const long f = d->cellFaces[6 * c + j];
-            const bool own = d->cellOwner[6 * c + j] != 0;
-            const double sgn = own ? 1.0 : -1.0;
-            const double w = d->weights[f];
-            for (int k = 0; k < 3; k++) sg[(size_t)(4 * j + k) * nIC + c] = (T)(sgn * (d->areas[f] * d->normals[3 * f + k]));
-            sg[(size_t)(4 * j + 3) * nIC + c] = (T)(own ? 1.0 - w : w);
+    std::vector<T> sn((size_t)24 * nPos, T(0)), tvol(nPos, T(1));
+    over_threads((int)(nPos / TILE_CELLS), [&](int a, int b) {
+        for (long p = (long)a * TILE_CELLS; p < (long)b * TILE_CELLS; p++) {
+            const long c = toUser[p];
+            if (c < 0) continue;
+            tvol[p] = (T)d->volumes[c];
+            for (int j = 0; j < 6; j++) {
+                const long f = d->cellFaces[6 * c + j];
+                const bool own = d->cellOwner[6 * c + j] != 0;
+                const double sgn = own ? 1.0 : -1.0;
+                const double w = d->weights[f];
+                for (int k = 0; k < 3; k++) sn[24 * p + 4 * j + k] = (T)(sgn * (d->areas[f] * d->normals[3 * f + k]));
+                sn[24 * p + 4 * j + 3] = (T)(own ? 1.0 - w : w);
+            }
         }
-    if ((rc = upload(ctx, &ctx->sgeo, sg)) != ADFVM_OK) return rc;
-    // The transposed gradient stencil for the gradient adjoint: cell c's
-    // slot j face value enters the gradient of the other side o with weight
-    // coef = (1 - w') and outward vector S*n_o, so d(grad_o)/d(w_c) through
-    // that face is coef * S*n_o / V_o.  Across an internal face that is
-    // -(1 - w') S*n_c / V_o (w' the other side's weight), which the kernel
-    // forms from the slot geometry; across a cyclic face it is the paired
-    // face fp seen from its owner o: S*n_fp and coef = 1 - w_fp, tabulated
-    // here.
-    std::vector<T> ng((size_t)18 * nIC, T(0));
-    for (long c = 0; c < nIC; c++)
-        for (int j = 0; j < 6; j++) {
-            const long f = d->cellFaces[6 * c + j];
-            if (f < ctx->nIF) continue;
-            const adfvm_patch_desc& Pd = d->patches[ctx->hBPatch[f - ctx->nIF]];
-            if (Pd.fluxKind != ADFVM_FLUX_COUPLED) continue;
-            const long g = d->patches[Pd.neighbourPatch].startFace + (f - Pd.startFace);
-            const long o = d->owner[g];
-            const double coef = 1.0 - d->weights[g];
-            for (int k = 0; k < 3; k++)
-                ng[(size_t)(3 * j + k) * nIC + c] = (T)(coef * (d->areas[g] * d->normals[3 * g + k]) / d->volumes[o]);
-        }
-    if ((rc = upload(ctx, &ctx->ngeo, ng)) != ADFVM_OK) return rc;
+    });
+    {
+        // the tables the blocks are filled from, freed at the end of the scope
+        struct Temp {
+            void* p[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
+            ~Temp() { for (void* q : p) if (q) (void)hipFree(q); }
+        } tmp;
+        if ((rc = upload(ctx, &tmp.p[0], sn)) != ADFVM_OK) return rc;
+        if ((rc = upload(ctx, &tmp.p[1], tvol)) != ADFVM_OK) return rc;
+        if ((rc = upload(ctx, &tmp.p[2], t.nbr)) != ADFVM_OK) return rc;
+        if ((rc = upload(ctx, &tmp.p[3], t.slots)) != ADFVM_OK) return rc;
+        if ((rc = upload(ctx, &tmp.p[4], t.halo)) != ADFVM_OK) return rc;
+        if ((rc = upload(ctx, &tmp.p[5], t.face)) != ADFVM_OK) return rc;
+        HIPCHK(ctx, hipMalloc((void**)&ctx->tileBlock, (size_t)ctx->nTiles * TileBlock<T>::BYTES));
+        HIPCHK(ctx, hipMalloc(&ctx->tileFaceW, ctx->nTileFaces() * sizeof(T)));
+        tile_block_kernel<T><<<ctx->nTiles, TILE_FACES>>>(
+            (const T*)ctx->geo, nF, (const T*)tmp.p[0], (const unsigned long long*)tmp.p[2],
+            (const unsigned long long*)tmp.p[3], (const int*)tmp.p[4], ctx->toUser, (const T*)tmp.p[1],
+            (const unsigned*)tmp.p[5], ctx->tileFaceId, ctx->tileBlock, (T*)ctx->tileFaceW);
+        HIPCHK(ctx, hipGetLastError());
+        HIPCHK(ctx, hipDeviceSynchronize());
+    }
     // boundary-condition values
     std::vector<T> vals;
     for (int p = 0; p < d->nPatches; p++) {
@@ -961,18 +746,17 @@ template <typename T> int create_typed(adfvm_ctx* ctx, const adfvm_solver_desc* 
     }
     if ((rc = upload(ctx, &ctx->bcval, vals)) != ADFVM_OK) return rc;
     // work buffers
-    size_t st = 5 * nIC * sizeof(T), gr = (size_t)GREC * nIC * sizeof(T);
+    const size_t st = 5 * nIC * sizeof(T), sp = 5 * nPos * sizeof(T);
     HIPCHK(ctx, hipMalloc(&ctx->ghost, std::max<size_t>(1, 5 * nBF) * sizeof(T)));
     HIPCHK(ctx, hipMemset(ctx->ghost, 0, std::max<size_t>(1, 5 * nBF) * sizeof(T)));
-    HIPCHK(ctx, hipMalloc(&ctx->u1, st));
-    HIPCHK(ctx, hipMalloc(&ctx->u2, st));
-    HIPCHK(ctx, hipMalloc(&ctx->grad0, gr));
-    HIPCHK(ctx, hipMalloc(&ctx->grad1, gr));
-    HIPCHK(ctx, hipMalloc(&ctx->grad2, gr));
-    HIPCHK(ctx, hipMalloc(&ctx->adjAcc, st));
-    HIPCHK(ctx, hipMalloc(&ctx->adjG, (size_t)AREC * nIC * sizeof(T)));
-    HIPCHK(ctx, hipMalloc(&ctx->fbuf, (size_t)FREC * nF * sizeof(T)));
-    HIPCHK(ctx, hipMalloc(&ctx->frec, (size_t)AREC * ctx->nPlanes * nIC * sizeof(T)));
+    for (int i = 0; i < 3; i++) {
+        HIPCHK(ctx, hipMalloc(&ctx->st[i], sp));
+        HIPCHK(ctx, hipMalloc(&ctx->rec[i], (size_t)CREC * nPos * sizeof(T)));
+    }
+    HIPCHK(ctx, hipMalloc(&ctx->rows1, st));
+    HIPCHK(ctx, hipMalloc(&ctx->adjU, sp));
+    HIPCHK(ctx, hipMalloc(&ctx->adjAcc, sp));
+    HIPCHK(ctx, hipMalloc(&ctx->adjG, (size_t)AREC * nPos * sizeof(T)));
     return ADFVM_OK;
 }
 
@@ -985,30 +769,15 @@ template <typename T> void launch_ghosts(adfvm_ctx* c, const T* u, hipStream_t s
     ghost_kernel<T><<<grid_for(c->nBF), BLOCK, 0, s>>>(dmesh<T>(c), phys_cast<T>(c->phd), u, P<T>(c->ghost));
 }
 
-template <typename T> void launch_grad(adfvm_ctx* c, const T* u, T* grad, hipStream_t s) {
+// Stage records of state u: the caller's rows (user) or state records; copy
+// (nullable): u as state records.
+template <typename T> void launch_grad(adfvm_ctx* c, const T* u, bool user, T* copy, T* rec, hipStream_t s) {
     KTimer kt(c, "grad_kernel", s);
-    with_block(c->bs[K_GRAD], [&](auto B) {
-        with_stream(c->stream, [&](auto S) {
-            with_ghosts(c->hasGhostKernel, [&](auto G) {
-                constexpr int BS = decltype(B)::value;
-                constexpr bool ST = decltype(S)::value, GH = decltype(G)::value;
-                grad_kernel<T, BS, ST, GH><<<grid_bs(c->nIC, BS), BS, 0, s>>>(dmesh<T>(c), phys_cast<T>(c->phd),
-                                                                               u, P<T>(c->ghost), grad);
-            });
-        });
-    });
-}
-
-template <typename T> void launch_face_flux(adfvm_ctx* c, const T* u, const T* grad, hipStream_t s) {
-    KTimer kt(c, "face_flux_kernel", s);
-    with_block(c->bs[K_FLUX], [&](auto B) {
-        with_stream(c->stream, [&](auto S) {
-            with_ghosts(c->hasGhostKernel, [&](auto G) {
-                constexpr int BS = decltype(B)::value;
-                constexpr bool ST = decltype(S)::value, GH = decltype(G)::value;
-                face_flux_kernel<T, BS, ST, GH><<<grid_bs(c->nF, BS), BS, 0, s>>>(
-                    dmesh<T>(c), phys_cast<T>(c->phd), u, grad, P<T>(c->ghost), P<T>(c->fbuf));
-            });
+    with_stream(c->stream, [&](auto SP) {
+        with_ghosts(c->hasGhostKernel, [&](auto G) {
+            constexpr bool ST = decltype(SP)::value, GH = decltype(G)::value;
+            grad_kernel<T, ST, GH><<<c->nTiles, TILE_CELLS, 0, s>>>(dmesh<T>(c), dtiles<T>(c),
+                                                                      phys_cast<T>(c->phd), u, user, copy, rec);
         });
     });
 }
@@ -1025,30 +794,21 @@ struct Stage {
     template <typename T> T a0_as() const { return a0 == 0.0 ? T(0) : T(1) - (T)ai; }
 };
 
+// Fluxes of all faces at the stage of records rec (state records u) and the
+// stage update into next (state records) and rows (the caller's), or the
+// residual.
 template <typename T, int MODE>
-void launch_stage(adfvm_ctx* c, const T* ui, const T* u0, const Stage& st, double dt, const T* S, T* out,
-                  T* dtcCell, double* dtcPartial, hipStream_t s) {
-    KTimer kt(c, MODE == 0 ? "stage_kernel" : "residual_kernel", s);
-    with_block(c->bs[K_STAGE], [&](auto B) {
-        with_stream(c->stream, [&](auto SP) {
-            constexpr int BS = decltype(B)::value;
-            constexpr bool ST = decltype(SP)::value;
-            stage_kernel<T, MODE, BS, ST><<<grid_bs(c->nIC, BS), BS, 0, s>>>(
-                dmesh<T>(c), P<T>(c->fbuf), ui, u0, (T)st.ai, (T)(-st.beta), (T)dt, S, out, dtcCell,
-                dtcPartial);
+void launch_flux_and_stage(adfvm_ctx* c, const T* rec, const T* u, const T* u0, const Stage& st, double dt,
+                           const T* S, T* next, T* rows, T* dtcCell, double* dtcPartial, hipStream_t s) {
+    KTimer kt(c, MODE == 0 ? "flux_stage_kernel" : "residual_kernel", s);
+    with_stream(c->stream, [&](auto SP) {
+        with_ghosts(c->hasGhostKernel, [&](auto G) {
+            constexpr bool ST = decltype(SP)::value, GH = decltype(G)::value;
+            flux_stage_kernel<T, MODE, ST, GH><<<c->nTiles, TILE_THREADS, 0, s>>>(
+                dmesh<T>(c), dtiles<T>(c), phys_cast<T>(c->phd), rec, u, u0, (T)st.ai, (T)(-st.beta), (T)dt, S, next,
+                rows, dtcCell, dtcPartial);
         });
     });
-}
-
-// Fluxes of all faces at state ui (gradients grad) and the stage update or
-// residual.  (A fused cell-centric variant that evaluates every face from
-// both sides instead of storing face records measured 2.3x slower: the face
-// flux is ALU-heavy.)
-template <typename T, int MODE>
-void launch_flux_and_stage(adfvm_ctx* c, const T* ui, const T* grad, const T* u0, const Stage& st, double dt,
-                           const T* S, T* out, T* dtcCell, double* dtcPartial, hipStream_t s) {
-    launch_face_flux<T>(c, ui, grad, s);
-    launch_stage<T, MODE>(c, ui, u0, st, dt, S, out, dtcCell, dtcPartial, s);
 }
 
 template <typename T> void launch_objective(adfvm_ctx* c, const T* u, double* out, hipStream_t s) {
@@ -1079,9 +839,6 @@ void stages(int integrator, std::vector<Stage>& st) {
     st.push_back({1.0 / 3.0, 2.0 / 3.0, 2.0 / 3.0});
 }
 
-// A step tape holds the forward step's intermediate stage states (all
-// stages but the first, whose state is the step's input) and every stage's
-// gradient records: [(ns-1) x 5 x nIC][ns x GREC x nIC] scalars.
 // The stage whose state the step's objective is evaluated on: the first
 // intermediate stage (density.py:412-413; the state a tape holds first), or
 // the step's start state u_n when the caller asked for it
@@ -1091,12 +848,16 @@ int objective_stage(const adfvm_ctx* c, int ns) {
     return (ns > 1 && c->objState == ADFVM_OBJSTATE_STAGE1) ? 1 : 0;
 }
 
-long tape_scalars(const adfvm_ctx* c, int ns) { return ((long)(ns - 1) * 5 + (long)ns * GREC) * c->nIC; }
+// A step tape holds the first intermediate stage's state in the caller's
+// numbering (schemes of several stages; what an objective of that stage
+// reads), then every stage's records: [5][nIC], [ns][nPos][CREC] scalars, both
+// from 16-byte boundaries of the tape.
+long tape_rows_scalars(const adfvm_ctx* c, int ns) { return ns > 1 ? (5L * c->nIC + 3) / 4 * 4 : 0; }
+long tape_scalars(const adfvm_ctx* c, int ns) { return tape_rows_scalars(c, ns) + (long)ns * CREC * c->nPos(); }
 
-template <typename T> void tape_slots(const adfvm_ctx* c, int ns, T* tape, T** states, T** grads) {
-    for (int i = 0; i < ns - 1; i++) states[i] = tape + (long)i * 5 * c->nIC;
-    T* g = tape + (long)(ns - 1) * 5 * c->nIC;
-    for (int i = 0; i < ns; i++) grads[i] = g + (long)i * GREC * c->nIC;
+template <typename T> void tape_slots(const adfvm_ctx* c, int ns, T* tape, T** rec) {
+    T* r = tape + tape_rows_scalars(c, ns);
+    for (int i = 0; i < ns; i++) rec[i] = r + (long)i * CREC * c->nPos();
 }
 
 template <typename T>
@@ -1105,27 +866,24 @@ int primal_step_t(adfvm_ctx* c, T* u, double dt, const T* S, double* dtc_out, do
     std::vector<Stage> st;
     stages(c->integrator, st);
     const int ns = (int)st.size();
-    T* bufs[3] = {P<T>(c->u1), P<T>(c->u2), u};
-    T* grads[3] = {P<T>(c->grad0), P<T>(c->grad1), P<T>(c->grad2)};
-    if (tape) tape_slots(c, ns, tape, bufs, grads);
-    const T* ui = u;
+    T* rec[3] = {P<T>(c->rec[0]), P<T>(c->rec[1]), P<T>(c->rec[2])};
+    if (tape) tape_slots(c, ns, tape, rec);
     const int objStage = objective_stage(c, ns);
     const int dtcStage = ns > 1 ? 1 : 0;    // density.py:412-413
+    // the objective stage's state in the caller's numbering, where one is needed
+    T* rows1 = ns == 1 ? nullptr : tape ? tape : (obj_out && objStage == 1) ? P<T>(c->rows1) : nullptr;
     for (int i = 0; i < ns; i++) {
-        // the last stage writes u in place (each cell reads only its own u0
-        // entry); a single-stage scheme reads u's neighbours, so it goes
-        // through u1 and is copied back
-        T* out = (i == ns - 1 && ns > 1) ? u : bufs[i];
-        if (i == objStage && obj_out) launch_objective<T>(c, ui, obj_out, s);
-        launch_grad<T>(c, ui, grads[i], s);
+        if (i == objStage && obj_out) launch_objective<T>(c, i == 0 ? u : rows1, obj_out, s);
+        launch_grad<T>(c, i == 0 ? u : P<T>(c->st[i]), i == 0, i == 0 ? P<T>(c->st[0]) : nullptr, rec[i], s);
         const bool wantDtc = (i == dtcStage) && dtc_out;
-        const T* u0 = (i > 0 && st[i].a0 != 0.0) ? (const T*)u : nullptr;
-        int g = grid_bs(c->nIC, c->bs[K_STAGE]);
-        launch_flux_and_stage<T, 0>(c, ui, grads[i], u0, st[i], dt, S, out, nullptr, wantDtc ? c->partial : nullptr, s);
-        if (wantDtc) finalize_kernel<1><<<1, BLOCK, 0, s>>>(c->partial, g, dtc_out);
-        ui = out;
+        const T* u0 = (i > 0 && st[i].a0 != 0.0) ? P<T>(c->st[0]) : nullptr;
+        // the last stage writes the caller's state in place: the kernels of
+        // this step read it no more (its records are st[0])
+        const bool last = i == ns - 1;
+        launch_flux_and_stage<T, 0>(c, rec[i], P<T>(c->st[i]), u0, st[i], dt, S, last ? nullptr : P<T>(c->st[i + 1]),
+                                    last ? u : i == 0 ? rows1 : nullptr, nullptr, wantDtc ? c->partial : nullptr, s);
+        if (wantDtc) finalize_kernel<1><<<1, BLOCK, 0, s>>>(c->partial, c->nTiles, dtc_out);
     }
-    if (ns == 1) copy_kernel<T><<<grid_for(5L * c->nIC), BLOCK, 0, s>>>(5L * c->nIC, bufs[0], u);
     HIPCHK(c, hipGetLastError());
     return ADFVM_OK;
 }
@@ -1238,13 +996,8 @@ extern "C" int adfvm_ctx_create(const adfvm_solver_desc* d, const adfvm_physics*
             fKind[f] = Pd.fluxKind == ADFVM_FLUX_CHARACTERISTIC ? FACE_CHARACTERISTIC : FACE_BOUNDARY;
         }
     }
-    // Face adjoint records sit in planes of nIC records: plane j holds, for
-    // every cell, the record of its slot j (its own side of an owned face,
-    // the neighbour side of a face it neighbours); planes 6, 7, ... hold, in
-    // slot order, the neighbour sides of the paired faces of a cell's cyclic
-    // slots (on which the cell is the ghost).  A cell's records for one slot
-    // are then at the same index of every plane, so neighbouring threads of
-    // the gather read neighbouring records.
+    // every face must have one slot per side; a cyclic face's neighbour side
+    // is the paired cell's, which takes it with its own slot (tiles.hpp)
     std::vector<int> posP(nF, -1), posN(nF, -1);
     int maxExtra = 0;
     for (long cc = 0; cc < nIC; cc++) {
@@ -1254,91 +1007,30 @@ extern "C" int adfvm_ctx_create(const adfvm_solver_desc* d, const adfvm_physics*
             const int f = sFace[j * nIC + cc];
             int& slot = (fl & 1) ? posP[f] : posN[f];
             if (slot != -1) return bad("face in two slots of the same side");
-            slot = (int)(j * nIC + cc);
+            slot = (int)cc;
             if (slot_kind(fl) == SLOT_COUPLED) e++;
         }
         maxExtra = std::max(maxExtra, e);
     }
     if ((long)(6 + maxExtra) * nIC > 0x7fffffffL) return bad("mesh too large for 32-bit record indices");
     for (long cc = 0; cc < nIC; cc++) {
-        int e = 0;
         for (int j = 0; j < 6; j++) {
             if (slot_kind(sFlags[j * nIC + cc]) != SLOT_COUPLED) continue;
             const int g = sPair[j * nIC + cc];
             if (posN[g] != -1) return bad("face with two neighbour-side slots");
-            posN[g] = (int)((6 + e++) * nIC + cc);
+            posN[g] = (int)cc;
         }
     }
     for (long f = 0; f < nF; f++) {
         if (posP[f] < 0) return bad("face without an owner slot");
         if (fKind[f] == FACE_INTERIOR && posN[f] < 0) return bad("face without a neighbour-side slot");
     }
-    c->nPlanes = 6 + maxExtra;
     int rc;
-    // the three groups: characteristic faces, boundary-kind faces whose
-    // ghost reads its patch, boundary-kind faces whose ghost copies the owner
-    std::vector<int> group(nBF, -1);
-    for (long b = 0; b < nBF; b++) {
-        if (fKind[nIF + b] == FACE_CHARACTERISTIC) group[b] = 0;
-        else if (fKind[nIF + b] == FACE_BOUNDARY) group[b] = ghost_copies_owner(d->patches[bPatch[b]]) ? 2 : 1;
-    }
-    for (int k = 0; k < 3; k++) {
-        std::vector<int> blk;                   // (first boundary index, count) per block
-        for (long b = 0; b < nBF;) {
-            if (group[b] != k) { b++; continue; }
-            long e = b;
-            while (e < nBF && group[e] == k) e++;
-            for (long b0 = b; b0 < e; b0 += BLOCK) {
-                blk.push_back((int)b0);
-                blk.push_back((int)std::min<long>(BLOCK, e - b0));
-            }
-            b = e;
-        }
-        c->nKindBlk[k] = (int)(blk.size() / 2);
-        if ((rc = upload(c, (void**)&c->kindBlk[k], blk)) != ADFVM_OK) return rc;
-    }
-    // The face adjoint sums a cell's owner sides in LDS when one owner's
-    // internal faces are consecutive (owners non-decreasing over the internal
-    // faces) and are the cell's first slots, in face order: the sum is then
-    // the gather's own sum over those slots.  Per block size, the face ranges
-    // end at owner changes.
-    c->ownerSum = true;
-    for (long f = 1; f < nIF && c->ownerSum; f++)
-        if (d->owner[f - 1] > d->owner[f]) c->ownerSum = false;
-    for (long cc = 0; cc < nIC && c->ownerSum; cc++) {
-        int prev = -1;
-        bool more = true;              // still in the leading run of owned internal slots
-        for (int j = 0; j < 6; j++) {
-            const int fl = sFlags[j * nIC + cc];
-            const bool ownInt = (fl & 1) && slot_kind(fl) == SLOT_INTERNAL;
-            if (ownInt && (!more || sFace[j * nIC + cc] <= prev)) { c->ownerSum = false; break; }
-            if (ownInt) prev = sFace[j * nIC + cc];
-            else more = false;
-        }
-    }
-    for (int k = 0; k < 4 && c->ownerSum; k++) {
-        const long bs = kBlockChoices[k];
-        std::vector<int> starts(1, 0);
-        for (long f = 0; f < nIF;) {
-            long e = std::min(f + bs, nIF);
-            while (e < nIF && e > f && d->owner[e - 1] == d->owner[e]) e--;
-            if (e == f) return bad("cell with more internal faces than a face adjoint block");
-            starts.push_back((int)e);
-            f = e;
-        }
-        c->fvjpNBlk[k] = (int)starts.size() - 1;
-        if ((rc = upload(c, (void**)&c->fvjpBlk[k], starts)) != ADFVM_OK) return rc;
-    }
-    if ((rc = upload(c, (void**)&c->posP, posP)) != ADFVM_OK) return rc;
-    if ((rc = upload(c, (void**)&c->posN, posN)) != ADFVM_OK) return rc;
     std::vector<int> owner(d->owner, d->owner + nF), nbFull(d->neighbour, d->neighbour + nF);
     if ((rc = upload(c, (void**)&c->fOther, fOther)) != ADFVM_OK) return rc;
-    {
-        std::vector<unsigned char> fKindDev(fKind);
-        for (long b = 0; b < nBF; b++)
-            if (ghost_copies_owner(d->patches[bPatch[b]])) fKindDev[nIF + b] |= FACE_GHOST_COPY;
-        if ((rc = upload(c, (void**)&c->fKind, fKindDev)) != ADFVM_OK) return rc;
-    }
+    for (long b = 0; b < nBF; b++)
+        if (ghost_copies_owner(d->patches[bPatch[b]])) fKind[nIF + b] |= FACE_GHOST_COPY;
+    if ((rc = upload(c, (void**)&c->fKind, fKind)) != ADFVM_OK) return rc;
     if ((rc = upload(c, (void**)&c->sFace, sFace)) != ADFVM_OK) return rc;
     if ((rc = upload(c, (void**)&c->sOther, sOther)) != ADFVM_OK) return rc;
     if ((rc = upload(c, (void**)&c->sFlags, sFlags)) != ADFVM_OK) return rc;
@@ -1348,11 +1040,23 @@ extern "C" int adfvm_ctx_create(const adfvm_solver_desc* d, const adfvm_physics*
     if ((rc = upload(c, (void**)&c->nbFull, nbFull)) != ADFVM_OK) return rc;
     if ((rc = upload(c, (void**)&c->bPatch, bPatch)) != ADFVM_OK) return rc;
     c->hBPatch = bPatch;
-    rc = c->prec == 4 ? create_typed<float>(c, d) : create_typed<double>(c, d);
-    if (rc != ADFVM_OK) return rc;
+    try {
+        Tiles t;
+        build_tiles(TileMesh{(int)nIC, (int)nIF, (int)nF, sFace.data(), sOther.data(), sPair.data(), sFlags.data(),
+                             fKind.data(), FACE_GHOST_COPY}, t);
+        c->nTiles = t.n;
+        if ((rc = upload(c, (void**)&c->toUser, t.toUser)) != ADFVM_OK) return rc;
+        if ((rc = upload(c, (void**)&c->toTile, t.toTile)) != ADFVM_OK) return rc;
+        if ((rc = upload(c, (void**)&c->tileFaceId, t.faceId)) != ADFVM_OK) return rc;
+        if ((rc = upload(c, (void**)&c->tilePairs, t.pairs)) != ADFVM_OK) return rc;
+        rc = c->prec == 4 ? create_typed<float>(c, d, t) : create_typed<double>(c, d, t);
+        if (rc != ADFVM_OK) return rc;
+    } catch (const std::exception& e) {
+        return bad(std::string("set-up of the mesh tables: ") + e.what());
+    }
     if ((rc = upload(c, (void**)&c->patches, c->hpatches)) != ADFVM_OK) return rc;
     c->stream = stream_auto(c);
-    c->nPartial = grid_bs(std::max<long>(nIC, nF), kBlockChoices[0]) + 1;   // the smallest block size
+    c->nPartial = std::max(grid_bs(std::max<long>(nIC, nF), kBlockChoices[0]) + 1, c->nTiles);   // the smallest block size
     HIPCHK(c, hipMalloc((void**)&c->partial, c->nPartial * sizeof(double)));
     HIPCHK(c, hipMalloc((void**)&c->scal, 16 * sizeof(double)));
     return ADFVM_OK;
@@ -1361,12 +1065,10 @@ extern "C" int adfvm_ctx_create(const adfvm_solver_desc* d, const adfvm_physics*
 extern "C" void adfvm_ctx_destroy(adfvm_ctx* c) {
     if (!c) return;
     void* ptrs[] = {c->geo, c->vol, c->bcval, c->sFace, c->sOther, c->sFlags, c->sPair, c->owner, c->bPatch,
-                    c->patches, c->cellNbFull, c->nbFull, c->ghost, c->u1, c->u2, c->grad0, c->grad1,
-                    c->grad2, c->adjAcc, c->adjG,
-                    c->partial, c->scal, c->fOther, c->fKind, c->fbuf, c->frec,
-                    c->segCell, c->segBlock, c->blockSeg, c->posP, c->posN, c->sgeo, c->ngeo, c->visc,
-                    c->fvjpBlk[0], c->fvjpBlk[1], c->fvjpBlk[2], c->fvjpBlk[3], c->kindBlk[0],
-                    c->kindBlk[1], c->kindBlk[2]};
+                    c->patches, c->cellNbFull, c->nbFull, c->ghost, c->st[0], c->st[1], c->st[2], c->rows1,
+                    c->rec[0], c->rec[1], c->rec[2], c->adjU, c->adjAcc, c->adjG,
+                    c->partial, c->scal, c->fOther, c->fKind, c->toUser, c->toTile, c->tileFaceId, c->tilePairs,
+                    c->tileBlock, c->tileFaceW, c->segCell, c->segBlock, c->blockSeg, c->visc};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     for (auto& p : c->pending) { (void)hipEventDestroy(p.a); (void)hipEventDestroy(p.b); }
@@ -1466,14 +1168,15 @@ extern "C" int adfvm_primal_step(adfvm_ctx* c, void* u, double dt, const void* S
 
 namespace {
 template <typename T> int gradients_t(adfvm_ctx* c, const T* u, T* grad, hipStream_t s) {
-    launch_grad<T>(c, u, P<T>(c->grad0), s);
-    grad_rows_kernel<T><<<grid_for(c->nIC), BLOCK, 0, s>>>(c->nIC, P<T>(c->grad0), grad);
+    launch_grad<T>(c, u, true, nullptr, P<T>(c->rec[0]), s);
+    grad_rows_kernel<T><<<grid_for(c->nIC), BLOCK, 0, s>>>(dtiles<T>(c), c->nIC, P<T>(c->rec[0]), grad);
     HIPCHK(c, hipGetLastError());
     return ADFVM_OK;
 }
 template <typename T> int residual_t(adfvm_ctx* c, const T* u, T* R, T* dtcCell, hipStream_t s) {
-    launch_grad<T>(c, u, P<T>(c->grad0), s);
-    launch_flux_and_stage<T, 1>(c, u, P<T>(c->grad0), nullptr, Stage{0, 0, 0}, 0.0, nullptr, R, dtcCell, nullptr, s);
+    launch_grad<T>(c, u, true, nullptr, P<T>(c->rec[0]), s);
+    launch_flux_and_stage<T, 1>(c, P<T>(c->rec[0]), nullptr, nullptr, Stage{0, 0, 0}, 0.0, nullptr, nullptr, R, dtcCell,
+                                nullptr, s);
     HIPCHK(c, hipGetLastError());
     return ADFVM_OK;
 }

@@ -34,28 +34,30 @@ HBM_PEAK = 8.0e12          # MI355X HBM3E, bytes/s
 
 def kernel_bytes(name, s, nC, nF, nG, nO=None):
     """Algorithmic bytes one launch moves: each array element the kernel
-    needs counted once (s = scalar bytes).  Cell slot tables: 6 x (int32
-    face, int32 neighbour, uint8 flags) = 54 B per cell, or 30 B without the
-    neighbour column; face tables: int32 owner + int32 neighbour + uint8 kind
-    = 9 B per face; the record indices of a face's adjoint (int32) 4 B per
-    record written by face.  Face adjoint records (20 scalars): with nO cells
-    owning internal faces (owner sides summed per cell) one per internal
-    face, one per such cell and two per cyclic face; otherwise two per face
-    (nO None).  Every boundary face here is cyclic (periodic box)."""
-    if name == 'grad_kernel':          # u, V, face (A, n, w) -> 15 gradients
-        return nC * (5 + 1 + 15) * s + nF * 5 * s + 54 * nC
-    if name == 'face_flux_kernel':     # u, grad, 16 face rows (all but the weight) -> 6 face values
-        return nC * (5 + 15) * s + nF * (16 + 6) * s + 9 * nF
-    if name == 'stage_kernel':         # face values, V, u_i, u0 (2 of 3 stages) -> u_{i+1}
-        return nF * 6 * s + nC * (1 + 5 + 10. / 3 + 5) * s + 30 * nC
+    needs counted once (s = scalar bytes).  The tile kernels read stage
+    records (5 primitives, 15 gradients), cell adjoint records (15 + 5) and,
+    per tile of about 64 cells, the geometry of its faces (16 rows, 4 B of
+    indices) or of its cells' slots (24 values), 24 B of indices per cell.
+    face_vjp_kernel and vjp_gather_kernel are a face kernel writing face
+    adjoint records (20 scalars) and the gather of them into cells: with nO
+    cells owning internal faces (owner sides summed per cell) one record per
+    internal face, one per such cell and two per cyclic face, otherwise two
+    per face (nO None); record indices (int32) 4 B per record written by face,
+    face tables 9 B per face, slot flags 6 B per cell."""
+    if name == 'grad_kernel':          # u, V, slot geometry -> stage records
+        return nC * (5 + 1 + 24 + 20) * s + 24 * nC
+    if name == 'flux_stage_kernel':    # stage records, face geometry, V, u_i, u0 (2 of 3 stages) -> u_{i+1}
+        return nC * (20 + 1 + 5 + 10. / 3 + 5) * s + nF * 16 * s + 4 * nF + 24 * nC
+    if name == 'flux_vjp_kernel':      # stage records, ubar, V, face geometry -> cell adjoint records
+        return nC * (20 + 5 + 1 + 20) * s + nF * 16 * s + 4 * nF + 24 * nC
+    if name == 'grad_vjp_kernel':      # w, cell adjoint records, ubar, acc (2 of 3), slot geometry -> ubar, acc
+        return nC * (5 + 20 + 5 + 10. / 3 + 24 + 5 + 10. / 3) * s + 24 * nC
     recs = 2 * nF if nO is None else (nF - nG) + nO + 2 * nG
     idx = 8 * nF if nO is None else 4 * (nF - nG) + 8 * nG
     if name == 'face_vjp_kernel':      # u, grad, ubar, V, 16 face rows -> face adjoint records
         return nC * (5 + 15 + 5 + 1) * s + nF * 16 * s + recs * 20 * s + 9 * nF + idx
     if name == 'vjp_gather_kernel':    # face adjoint records -> wbar, gbar; slot flags
         return recs * 20 * s + nC * 20 * s + 6 * nC
-    if name == 'grad_vjp_kernel':      # u, wbar, gbar, ubar, acc (2 of 3), V, 6 x 4 slot coefficients -> ubar, acc
-        return nC * (5 + 5 + 15 + 5 + 10. / 3 + 1 + 5 + 10. / 3 + 24) * s + 30 * nC
     return None
 
 
@@ -91,7 +93,7 @@ def run_precision(case, u0, prec, K, W, dt, torch, profile, recompute=False):
     ctx = case.context(prec)
     nC = ctx.nIC
     u = torch.as_tensor(u0.astype(prec), device='cuda').contiguous()
-    tuned = ctx.autotune(u, reps=3)          # block size per stencil kernel (results do not depend on it)
+    tuned = ctx.autotune(u, reps=3)          # times the stencil kernels
     store = torch.empty((K, 5, nC), dtype=ctx.tdtype, device='cuda')
     tapes = None if recompute else ctx.new_tapes(K)
     ua = torch.zeros_like(u)

@@ -241,13 +241,14 @@ int adfvm_objective_state(const adfvm_ctx* ctx);
  * first intermediate stage, density.py:405-413.  obj_out (device double,
  * nullable): the objective on the same stage (or on u_n, see
  * adfvm_set_objective_state), in FP64.  tape (device,
- * adfvm_tape_bytes() bytes, nullable): receives the step's intermediate
- * stage states and stage gradients for a later adfvm_adjoint_step. */
+ * adfvm_tape_bytes() bytes, nullable): receives the first intermediate stage's
+ * state ([5][nIC], schemes of several stages) and, in the library's own layout,
+ * every stage's values and gradients for a later adfvm_adjoint_step. */
 int adfvm_primal_step(adfvm_ctx* ctx, void* u, double dt, const void* source,
                       double* dtc_out, double* obj_out, void* tape, void* stream);
 
-/* Size in bytes of one step's tape (2 stage states + 3 stage gradient
- * records for SSP-RK3).  Keeping tapes trades HBM capacity for the forward
+/* Size in bytes of one step's tape (one stage state + 3 records of 20 scalars
+ * per cell for SSP-RK3).  Keeping tapes trades HBM capacity for the forward
  * recomputation the reference's reverse sweep does (apps/adjoint.py:211-217). */
 int64_t adfvm_tape_bytes(const adfvm_ctx* ctx);
 
@@ -321,21 +322,21 @@ int adfvm_set_mesh_grad(adfvm_ctx* ctx, void* mesh_grad);
 int adfvm_adjoint_viscosity(adfvm_ctx* ctx, const void* u_n, void* ua, double dt, int32_t type, double scaling,
                             int32_t iterations, void* m2norm_out, void* stream);
 
-/* Block-size autotuner for the six stencil kernels (gradient, face flux,
- * stage update, face adjoint, adjoint gather, gradient adjoint).  Times each
- * at 64, 128, 256 and 512 threads per block (reps timed launches each) on
- * the device state u and keeps the fastest for this context.  Results do not
- * depend on the block size: each thread's arithmetic is unchanged and the
- * only cross-thread combination in these kernels is a maximum.  Uses the
- * context's work buffers and synchronizes the stream, so it is not for use
- * inside graph capture.  No counterpart in the reference (adpy fixes its
- * launch shapes at code generation). */
+/* Times the stencil kernels (reps timed launches each) on the device state u.
+ * The kernels work on tiles of up to 64 cells, which fix their blocks, so
+ * there is no block size to choose; the six names are kept: face_flux_kernel
+ * and stage_kernel are one kernel (fluxes and stage update), face_vjp_kernel
+ * and vjp_gather_kernel another (their transpose), and each name reports its
+ * kernel's time.  Uses the context's work buffers and synchronizes the stream,
+ * so it is not for use inside graph capture.  No counterpart in the reference
+ * (adpy fixes its launch shapes at code generation). */
 int adfvm_autotune(adfvm_ctx* ctx, const void* u, int32_t reps, void* stream);
-/* i-th tunable kernel (0 <= i < 6): its name, the block size in use and the
- * time per launch adfvm_autotune measured for it (-1 if not tuned). */
+/* i-th stencil kernel name (0 <= i < 6), its block size (256) and the time per
+ * launch adfvm_autotune measured for it (-1 before). */
 int adfvm_kernel_config(const adfvm_ctx* ctx, int32_t i, char* name, int32_t len, int32_t* block,
                         double* ms);
-/* Sets one tunable kernel's block size (64, 128, 256 or 512) by name. */
+/* Accepts a block size (64, 128, 256 or 512) for a stencil kernel's name; the
+ * tiles fix the blocks, so it changes nothing. */
 int adfvm_set_kernel_block(adfvm_ctx* ctx, const char* name, int32_t block);
 /* Streaming policy of the stencil kernels: mode 1 loads the rows a launch
  * uses once (face and slot geometry, slot tables, a cell's own state)
