@@ -500,6 +500,14 @@ __global__ void __launch_bounds__(BLOCK) copy_kernel(long n, const T* __restrict
 
 // ----------------------------------------------------------- context -----
 
+// A local cell of a patch (viscosity.inc): its position, and the local cell
+// across each slot's face.
+struct RingCell {
+    int pos;
+    unsigned short nbr[6];
+};
+static_assert(sizeof(RingCell) == 16, "one 16-byte load");
+
 struct adfvm_ctx {
     int prec = 4;
     int nIC = 0, nIF = 0, nF = 0, nBF = 0, nC = 0;
@@ -519,7 +527,14 @@ struct adfvm_ctx {
     int* cellNbFull = nullptr;   // reference cellNeighbours [6][nIC]
     int* nbFull = nullptr;       // ghost-extended neighbour [nF]
     void* ghost = nullptr;
-    void* visc = nullptr;      // adjoint viscosity: [6][nIC] slot coefficients, [nIC] diagonal, [nIC] eigenvalue
+    // adjoint viscosity, from its first call on: [6][nIC] slot coefficients,
+    // [nIC] diagonal, [nIC] eigenvalue; the patches' tables (sweeps at a time,
+    // patches) and [nPos][12] slot coefficients, diagonal, right side
+    void* visc = nullptr;
+    int ringK = 1, ringN = 0;
+    RingCell* ringCell = nullptr;
+    int* ringCount = nullptr;
+    void* ringCoef = nullptr;
     void* st[3] = {nullptr, nullptr, nullptr};    // state records of the step's start and its intermediate stages
     void* rows1 = nullptr;     // [5][nIC] the objective stage's state in the caller's numbering
     void* rec[3] = {nullptr, nullptr, nullptr};   // [nIC][CREC] stage records
@@ -1068,7 +1083,7 @@ extern "C" void adfvm_ctx_destroy(adfvm_ctx* c) {
                     c->patches, c->cellNbFull, c->nbFull, c->ghost, c->st[0], c->st[1], c->st[2], c->rows1,
                     c->rec[0], c->rec[1], c->rec[2], c->adjU, c->adjAcc, c->adjG,
                     c->partial, c->scal, c->fOther, c->fKind, c->toUser, c->toTile, c->tileFaceId, c->tilePairs,
-                    c->tileBlock, c->tileFaceW, c->segCell, c->segBlock, c->blockSeg, c->visc};
+                    c->tileBlock, c->tileFaceW, c->segCell, c->segBlock, c->blockSeg, c->visc, c->ringCell, c->ringCount, c->ringCoef};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     for (auto& p : c->pending) { (void)hipEventDestroy(p.a); (void)hipEventDestroy(p.b); }
