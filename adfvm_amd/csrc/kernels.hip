@@ -505,14 +505,6 @@ __global__ void __launch_bounds__(BLOCK) copy_kernel(long n, const T* __restrict
 
 // ----------------------------------------------------------- context -----
 
-// A local cell of a patch (viscosity.inc): its position, and the local cell
-// across each slot's face.
-struct RingCell {
-    int pos;
-    unsigned short nbr[6];
-};
-static_assert(sizeof(RingCell) == 16, "one 16-byte load");
-
 struct adfvm_ctx {
     int prec = 4;
     int nIC = 0, nIF = 0, nF = 0, nBF = 0, nC = 0;
@@ -561,6 +553,7 @@ struct adfvm_ctx {
     int nTiles = 0;
     long nPos() const { return (long)TILE_CELLS * nTiles; }
     long nTileFaces() const { return (long)TILE_FACES * nTiles; }
+    TileRing* tileRing = nullptr;   // [nTiles], null: stages in two launches
     int* toUser = nullptr; int* toTile = nullptr; int* tileFaceId = nullptr;
     unsigned long long* tilePairs = nullptr;
     unsigned char* tileBlock = nullptr; void* tileFaceW = nullptr;
@@ -670,10 +663,16 @@ template <typename T> DMesh<T> dmesh(const adfvm_ctx* c) {
 template <typename T> DTiles<T> dtiles(const adfvm_ctx* c) {
     DTiles<T> t;
     t.n = c->nTiles;
-    t.block = c->tileBlock; t.toUser = c->toUser; t.toTile = c->toTile; t.faceId = c->tileFaceId; t.pairs = c->tilePairs;
+    t.ring = c->tileRing; t.block = c->tileBlock; t.toUser = c->toUser; t.toTile = c->toTile; t.faceId = c->tileFaceId; t.pairs = c->tilePairs;
     t.faceW = (const T*)c->tileFaceW;
     return t;
 }
+
+// The most tiles for which a stage takes one launch (20 a compute unit), and one
+// whose records are kept: 4, or 1 where a compute unit holds two blocks only
+// (FP64 with ghosts: 69 KB of LDS).  Measured at launch_stage.
+constexpr int ONE_LAUNCH_TILES = 5120;
+int one_launch_rec_tiles(const adfvm_ctx* c) { return c->prec == 8 && c->hasGhostKernel ? 256 : 1024; }
 
 template <typename T> int upload(adfvm_ctx* ctx, void** dst, const std::vector<T>& v) {
     HIPCHK(ctx, hipMalloc(dst, std::max<size_t>(1, v.size()) * sizeof(T)));
@@ -727,7 +726,7 @@ template <typename T> int create_typed(adfvm_ctx* ctx, const adfvm_solver_desc* 
     {
         // the tables the blocks are filled from, freed at the end of the scope
         struct Temp {
-            void* p[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
+            void* p[7] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
             ~Temp() { for (void* q : p) if (q) (void)hipFree(q); }
         } tmp;
         if ((rc = upload(ctx, &tmp.p[0], sn)) != ADFVM_OK) return rc;
@@ -743,6 +742,22 @@ template <typename T> int create_typed(adfvm_ctx* ctx, const adfvm_solver_desc* 
             (const unsigned long long*)tmp.p[3], (const int*)tmp.p[4], ctx->toUser, (const T*)tmp.p[1],
             (const unsigned*)tmp.p[5], ctx->tileFaceId, ctx->tileBlock, (T*)ctx->tileFaceW);
         HIPCHK(ctx, hipGetLastError());
+        // the rings around the tiles, where stages are to take one launch
+        // (launch_stage): not where one does not fit, or the memory for them is
+        // not to be had
+        if (ctx->nTiles <= ONE_LAUNCH_TILES &&
+            hipMalloc((void**)&ctx->tileRing, (size_t)ctx->nTiles * sizeof(TileRing)) == hipSuccess) {
+            int over = 0;
+            if ((rc = upload(ctx, &tmp.p[6], std::vector<int>(1, 0))) != ADFVM_OK) return rc;
+            tile_ring_kernel<<<ctx->nTiles, TILE_HALO>>>(nIC, (const int*)tmp.p[4], ctx->toUser, ctx->toTile, ctx->sOther,
+                                                         ctx->sFace, ctx->fKind, ctx->tileRing, (int*)tmp.p[6]);
+            HIPCHK(ctx, hipGetLastError());
+            HIPCHK(ctx, hipMemcpy(&over, tmp.p[6], sizeof(int), hipMemcpyDeviceToHost));
+            if (over) { (void)hipFree(ctx->tileRing); ctx->tileRing = nullptr; }
+        } else {
+            (void)hipGetLastError();
+            ctx->tileRing = nullptr;
+        }
         HIPCHK(ctx, hipDeviceSynchronize());
     }
     // boundary-condition values
@@ -831,6 +846,42 @@ void launch_flux_and_stage(adfvm_ctx* c, const T* rec, const T* u, const T* u0, 
     });
 }
 
+// Gradients, fluxes and the stage update (or the residual): one launch, or two
+// through the records work.  u: the caller's rows (user) or state records,
+// copy (nullable): its records, which the update reads; rec (nullable): where
+// the stage's records are kept.
+// One launch saves a launch and, where records are not kept, their way through
+// memory; it forms a halo cell's gradients again in every tile beside it (2.5
+// times the gradient work, from 2.6 times the slot geometry).  Steps in us,
+// two -> one launches: 1000 cells in a tube FP64 44.3 -> 39.7, 32^3 FP64 70.5 ->
+// 66.8, 48^3 75.9 -> 71.4 (FP64 129.5 -> 119.2), 64^3 (4.2k tiles) 129.9 -> 126.5
+// (FP64 273 -> 245), 80^3 (8k tiles) 248 -> 259, 101x83x67 269 -> 279.  Steps that
+// keep records with their adjoint steps: 16^3 63.3 -> 57.8, 48^3 (1.8k tiles) 160.5
+// -> 159.8, 64^3 292 -> 296; cells of an O-grid 8.6k 86 -> 79, 33k 104 -> 100 (FP64
+// 104 -> 96, 168 -> 168), a duct of 25k FP64 156 -> 159.  Two launches also where a tile's ring does not fit
+// and where the rows written are those read.
+template <typename T, int MODE>
+void launch_stage(adfvm_ctx* c, const T* u, bool user, T* copy, T* rec, T* work, const T* u0, const Stage& st, double dt,
+                  const T* S, T* next, T* rows, T* dtcCell, double* dtcPartial, hipStream_t s) {
+    auto over_u = [&](const T* out, long n) { return user && out && out < u + 5L * c->nIC && u < out + n; };
+    const bool overlap = over_u(rows, 5L * c->nIC) || over_u(dtcCell, c->nIC);
+    if (!c->tileRing || overlap || (rec && c->nTiles > one_launch_rec_tiles(c))) {
+        T* r = rec ? rec : work;
+        launch_grad<T>(c, u, user, copy, r, s);
+        launch_flux_and_stage<T, MODE>(c, r, user ? copy : u, u0, st, dt, S, next, rows, dtcCell, dtcPartial, s);
+        return;
+    }
+    KTimer kt(c, MODE == 0 ? "tile_stage_kernel" : "tile_residual_kernel", s);
+    with_stream(c->stream, [&](auto SP) {
+        with_ghosts(c->hasGhostKernel, [&](auto G) {
+            constexpr bool ST = decltype(SP)::value, GH = decltype(G)::value;
+            tile_stage_kernel<T, MODE, ST, GH><<<c->nTiles, TILE_THREADS, 0, s>>>(
+                dmesh<T>(c), dtiles<T>(c), phys_cast<T>(c->phd), u, user, copy, rec, u0, (T)st.ai, (T)(-st.beta), (T)dt, S,
+                next, rows, dtcCell, dtcPartial);
+        });
+    });
+}
+
 template <typename T> void launch_objective(adfvm_ctx* c, const T* u, double* out, hipStream_t s) {
     KTimer kt(c, "objective", s);
     if (c->objective == ADFVM_OBJ_KINETIC_ENERGY && c->nSeg > 1) {
@@ -894,14 +945,14 @@ int primal_step_t(adfvm_ctx* c, T* u, double dt, const T* S, double* dtc_out, do
     T* rows1 = ns == 1 ? nullptr : tape ? tape : (obj_out && objStage == 1) ? P<T>(c->rows1) : nullptr;
     for (int i = 0; i < ns; i++) {
         if (i == objStage && obj_out) launch_objective<T>(c, i == 0 ? u : rows1, obj_out, s);
-        launch_grad<T>(c, i == 0 ? u : P<T>(c->st[i]), i == 0, i == 0 ? P<T>(c->st[0]) : nullptr, rec[i], s);
         const bool wantDtc = (i == dtcStage) && dtc_out;
         const T* u0 = (i > 0 && st[i].a0 != 0.0) ? P<T>(c->st[0]) : nullptr;
         // the last stage writes the caller's state in place: the kernels of
         // this step read it no more (its records are st[0])
         const bool last = i == ns - 1;
-        launch_flux_and_stage<T, 0>(c, rec[i], P<T>(c->st[i]), u0, st[i], dt, S, last ? nullptr : P<T>(c->st[i + 1]),
-                                    last ? u : i == 0 ? rows1 : nullptr, nullptr, wantDtc ? c->partial : nullptr, s);
+        launch_stage<T, 0>(c, i == 0 ? u : P<T>(c->st[i]), i == 0, i == 0 ? P<T>(c->st[0]) : nullptr,
+                           tape ? rec[i] : nullptr, P<T>(c->rec[i]), u0, st[i], dt, S, last ? nullptr : P<T>(c->st[i + 1]),
+                           last ? u : i == 0 ? rows1 : nullptr, nullptr, wantDtc ? c->partial : nullptr, s);
         if (wantDtc) finalize_kernel<1><<<1, FINAL_THREADS<1>, 0, s>>>(c->partial, c->nTiles, dtc_out);
     }
     HIPCHK(c, hipGetLastError());
@@ -1088,7 +1139,7 @@ extern "C" void adfvm_ctx_destroy(adfvm_ctx* c) {
                     c->patches, c->cellNbFull, c->nbFull, c->ghost, c->st[0], c->st[1], c->st[2], c->rows1,
                     c->rec[0], c->rec[1], c->rec[2], c->adjU, c->adjAcc, c->adjG,
                     c->partial, c->scal, c->fOther, c->fKind, c->toUser, c->toTile, c->tileFaceId, c->tilePairs,
-                    c->tileBlock, c->tileFaceW, c->segCell, c->segBlock, c->blockSeg, c->visc, c->ringCell, c->ringCount, c->ringCoef};
+                    c->tileBlock, c->tileRing, c->tileFaceW, c->segCell, c->segBlock, c->blockSeg, c->visc, c->ringCell, c->ringCount, c->ringCoef};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     for (auto& p : c->pending) { (void)hipEventDestroy(p.a); (void)hipEventDestroy(p.b); }
@@ -1194,9 +1245,8 @@ template <typename T> int gradients_t(adfvm_ctx* c, const T* u, T* grad, hipStre
     return ADFVM_OK;
 }
 template <typename T> int residual_t(adfvm_ctx* c, const T* u, T* R, T* dtcCell, hipStream_t s) {
-    launch_grad<T>(c, u, true, nullptr, P<T>(c->rec[0]), s);
-    launch_flux_and_stage<T, 1>(c, P<T>(c->rec[0]), nullptr, nullptr, Stage{0, 0, 0}, 0.0, nullptr, nullptr, R, dtcCell,
-                                nullptr, s);
+    launch_stage<T, 1>(c, u, true, nullptr, nullptr, P<T>(c->rec[0]), nullptr, Stage{0, 0, 0}, 0.0, nullptr, nullptr, R,
+                       dtcCell, nullptr, s);
     HIPCHK(c, hipGetLastError());
     return ADFVM_OK;
 }
