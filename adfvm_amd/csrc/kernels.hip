@@ -708,7 +708,7 @@ template <typename T> int create_typed(adfvm_ctx* ctx, const adfvm_solver_desc* 
     // (phi_f = phi_c (1 - w') + phi_other w'), streamed by the gradient
     // kernels instead of gathering face rows.
     std::vector<T> sn((size_t)24 * nPos, T(0)), tvol(nPos, T(1));
-    over_threads((int)(nPos / TILE_CELLS), [&](int a, int b) {
+    over_threads((int)(nPos / TILE_CELLS), [&](int a, int b, int) {
         for (long p = (long)a * TILE_CELLS; p < (long)b * TILE_CELLS; p++) {
             const long c = toUser[p];
             if (c < 0) continue;

@@ -66,10 +66,58 @@ struct Tiles {
     std::vector<uint64_t> slots, pairs, nbr;   // [n][TILE_CELLS] cell words
 };
 
+// The parts over_threads splits [0, n) into.
+inline int thread_parts(int n) { return std::max(1, std::min({8, (int)std::thread::hardware_concurrency(), n / 64})); }
+
+// f(a, b, k) over the parts k of [0, n), a host thread each; a part whose
+// thread cannot be started runs on this one, and the first exception of any
+// part is rethrown here when all have ended.
+template <typename F> void over_threads(int n, F&& f) {
+    const int nt = thread_parts(n);
+    std::vector<std::exception_ptr> err(nt);
+    auto part = [&](int k) {
+        try {
+            f((int)((long)n * k / nt), (int)((long)n * (k + 1) / nt), k);
+        } catch (...) {
+            err[k] = std::current_exception();
+        }
+    };
+    std::vector<std::thread> th;
+    th.reserve(nt);
+    for (int k = 1; k < nt; k++) {
+        try {
+            th.emplace_back(part, k);
+        } catch (const std::system_error&) {
+            part(k);
+        }
+    }
+    part(0);
+    for (auto& x : th) x.join();
+    for (auto& e : err)
+        if (e) std::rethrow_exception(e);
+}
+
+// A cell's six neighbours in one place, n cells: the other cell, or -2 - cell
+// across a cyclic face, or -1 (a ghost).  The slot tables are rows of all
+// cells, six cache lines for a cell.
+inline std::vector<int> neighbour_list(const TileMesh& m) {
+    const long n = m.nIC;
+    std::vector<int> near(6 * n);
+    over_threads(m.nIC, [&](int a, int b, int) {
+        for (long c = a; c < b; c++)
+            for (int j = 0; j < 6; j++) {
+                const int o = m.sOther[j * n + c];
+                near[6 * c + j] = o < 0 ? -1 : m.sPair[j * n + c] >= 0 ? -2 - o : o;
+            }
+    });
+    return near;
+}
+
 // Grows the tiles: tileOf order as lists of own cells, ascending in each.
 // Candidates wait in one queue per number of neighbours inside (oldest
 // first); stale entries are skipped when they come up.
-inline void grow_tiles(const TileMesh& m, std::vector<int>& cells, std::vector<int>& start) {
+inline void grow_tiles(const TileMesh& m, const std::vector<int>& near, std::vector<int>& cells,
+                       std::vector<int>& start) {
     const long n = m.nIC;
     std::vector<char> taken(n, 0);
     std::vector<int> gain(n, 0), gainTile(n, -1), nearTile(n, -1);
@@ -102,9 +150,8 @@ inline void grow_tiles(const TileMesh& m, std::vector<int>& cells, std::vector<i
             int df = 0, dh = nearTile[c] == tile ? -1 : 0;
             int fresh[6], nFresh = 0;
             for (int j = 0; j < 6; j++) {
-                const int o = m.sOther[j * n + c];
-                const bool cyclic = m.sPair[j * n + c] >= 0;
-                if (cyclic) df += 2;
+                const int e = near[6L * c + j], o = e < -1 ? -2 - e : e;
+                if (e < -1) df += 2;
                 else if (o < 0) df += 1;
                 else if (nearTile[o] != -2 - tile) df += 1;
                 if (o >= 0 && o != c && nearTile[o] != tile && nearTile[o] != -2 - tile) {
@@ -123,8 +170,8 @@ inline void grow_tiles(const TileMesh& m, std::vector<int>& cells, std::vector<i
             cells.push_back(c);
             for (int k = 0; k < nFresh; k++) nearTile[fresh[k]] = tile;
             for (int j = 0; j < 6; j++) {
-                const int o = m.sOther[j * n + c];
-                if (o < 0 || m.sPair[j * n + c] >= 0 || taken[o]) continue;
+                const int o = near[6L * c + j];
+                if (o < 0 || taken[o]) continue;
                 if (gainTile[o] != tile) { gainTile[o] = tile; gain[o] = 0; }
                 queue[++gain[o]].push_back(o);
             }
@@ -142,7 +189,8 @@ inline void grow_tiles(const TileMesh& m, std::vector<int>& cells, std::vector<i
 // through its cache.  In growth order a layer of tiles spans the whole mesh
 // before the next begins, and every halo came from memory: at 128^3 FP32 the
 // four kernels of a stage and its reverse read 3.92 GB, in this order 3.01 GB.
-inline void order_tiles(const TileMesh& m, std::vector<int>& cells, std::vector<int>& start) {
+inline void order_tiles(const TileMesh& m, const std::vector<int>& near, std::vector<int>& cells,
+                        std::vector<int>& start) {
     const long n = m.nIC;
     int nodes = (int)start.size() - 1;
     const int nt = nodes;
@@ -160,23 +208,28 @@ inline void order_tiles(const TileMesh& m, std::vector<int>& cells, std::vector<
         e.resize(k);
     };
     std::vector<Edge> edges;
-    for (int t = 0; t < nt; t++) {
-        const size_t first = edges.size();
-        for (int i = start[t]; i < start[t + 1]; i++)
-            for (int j = 0; j < 6; j++) {
-                const int o = m.sOther[j * n + cells[i]];
-                if (o < 0 || node[o] == t) continue;
-                bool seen = false;
-                for (size_t k = first; k < edges.size() && !seen; k++)
-                    if (edges[k].b == node[o]) { edges[k].w++; seen = true; }
-                if (!seen) edges.push_back({t, node[o], 1});
-            }
-    }
+    std::vector<std::vector<Edge>> part(thread_parts(nt));
+    over_threads(nt, [&](int a, int b, int p) {
+        std::vector<Edge>& e = part[p];
+        for (int t = a; t < b; t++) {
+            const size_t first = e.size();
+            for (int i = start[t]; i < start[t + 1]; i++)
+                for (int j = 0; j < 6; j++) {
+                    const int x = near[6L * cells[i] + j], o = x < -1 ? -2 - x : x;
+                    if (o < 0 || node[o] == t) continue;
+                    bool seen = false;
+                    for (size_t k = first; k < e.size() && !seen; k++)
+                        if (e[k].b == node[o]) { e[k].w++; seen = true; }
+                    if (!seen) e.push_back({t, node[o], 1});
+                }
+        }
+    });
+    for (const auto& e : part) edges.insert(edges.end(), e.begin(), e.end());
     std::vector<std::vector<int>> leaves(nt);        // a node's tiles in order
     for (int t = 0; t < nt; t++) leaves[t] = {t};
     while (nodes > 1) {
         merge(edges);
-        std::vector<int> first(nodes + 1, 0), group(nodes, -1), weight(nodes, 0), mark(nodes, -1), near;
+        std::vector<int> first(nodes + 1, 0), group(nodes, -1), weight(nodes, 0), mark(nodes, -1), beside;
         for (const Edge& e : edges) first[e.a + 1]++;
         for (int k = 0; k < nodes; k++) first[k + 1] += first[k];
         std::vector<std::vector<int>> up;
@@ -184,18 +237,18 @@ inline void order_tiles(const TileMesh& m, std::vector<int>& cells, std::vector<
             if (group[seed] >= 0) continue;
             const int g = (int)up.size();
             up.emplace_back();
-            near.clear();
+            beside.clear();
             for (int c = seed, size = 0; c >= 0 && size < 8; size++) {
                 group[c] = g;
                 up[g].insert(up[g].end(), leaves[c].begin(), leaves[c].end());
                 for (int e = first[c]; e < first[c + 1]; e++) {
                     const int o = edges[e].b;
                     if (group[o] >= 0) continue;
-                    if (mark[o] != g) { mark[o] = g; weight[o] = 0; near.push_back(o); }
+                    if (mark[o] != g) { mark[o] = g; weight[o] = 0; beside.push_back(o); }
                     weight[o] += edges[e].w;
                 }
                 c = -1;
-                for (int o : near)
+                for (int o : beside)
                     if (group[o] < 0 && (c < 0 || weight[o] > weight[c])) c = o;
             }
         }
@@ -219,80 +272,86 @@ inline void order_tiles(const TileMesh& m, std::vector<int>& cells, std::vector<
     start.swap(start2);
 }
 
-// One tile's lists, found by sorting, so tiles are independent of one another.
-struct TileLists {
-    std::vector<int> halo, pair, inter, ghost;   // ascending (ghost: by kind, then ascending)
+// Numbers small integers in the order they are first given (open addressing;
+// at most half full).
+struct Numbering {
+    static constexpr int SIZE = 1024;
+    int key[SIZE], value[SIZE];
+    void clear() { std::fill(key, key + SIZE, -1); }
+    int* find(int k) {                 // k's entry, or the free one where it goes
+        unsigned h = (unsigned)k * 2654435761u >> 22;
+        while (key[h] != -1 && key[h] != k) h = (h + 1) & (SIZE - 1);
+        return &key[h];
+    }
+    int at(int k) { return value[find(k) - key]; }
+    bool add(int k, int v) {           // false: k is there already
+        int* p = find(k);
+        if (*p == k) return false;
+        *p = k;
+        value[p - key] = v;
+        return true;
+    }
 };
 
-inline int index_in(const std::vector<int>& v, int x) {      // x's place in the ascending v, or -1
-    const auto p = std::lower_bound(v.begin(), v.end(), x);
-    return p != v.end() && *p == x ? (int)(p - v.begin()) : -1;
-}
-
-inline void list_tile(const TileMesh& m, const Tiles& out, int tile, int nOwn, TileLists& t) {
-    const long n = m.nIC;
-    t.halo.clear(); t.pair.clear(); t.inter.clear(); t.ghost.clear();
-    auto unique = [](std::vector<int>& v) {
-        std::sort(v.begin(), v.end());
-        v.erase(std::unique(v.begin(), v.end()), v.end());
-    };
-    const int* own = out.toUser.data() + (size_t)tile * TILE_CELLS;
-    for (int i = 0; i < nOwn; i++)
-        for (int j = 0; j < 6; j++) {
-            const long s = j * n + own[i];
-            const int o = m.sOther[s];
-            if (o < 0) { t.ghost.push_back(m.sFace[s]); continue; }
-            t.inter.push_back(m.sFace[s]);
-            const int p = out.toTile[o];
-            if (p / TILE_CELLS != tile) t.halo.push_back(p);
-        }
-    unique(t.halo);
-    unique(t.inter);
-    for (int i = 0; i < nOwn; i++)
-        for (int j = 0; j < 6; j++) {
-            const int g = m.sPair[j * n + own[i]];
-            if (g >= 0 && index_in(t.inter, g) < 0) t.pair.push_back(g);
-        }
-    unique(t.pair);
-    std::sort(t.ghost.begin(), t.ghost.end(), [&](int a, int b) {
-        return m.fKind[a] != m.fKind[b] ? m.fKind[a] < m.fKind[b] : a < b;
-    });
-}
-
-// Writes a tile's lists and words.  Faces in order: the cells' internal and
-// cyclic faces, the paired faces of cyclic slots (whose neighbour side the
-// cell takes), the faces with a ghost by kind.
-inline void fill_tile(const TileMesh& m, int tile, int nOwn, const TileLists& t, Tiles& out) {
+// Lists a tile and writes its words.  Faces in order: the cells' internal and
+// cyclic faces as their slots come, the paired faces of cyclic slots (whose
+// neighbour side the cell takes), the faces with a ghost by kind.  A tile has at
+// most TILE_FACES faces and TILE_HALO halo cells.
+inline void fill_tile(const TileMesh& m, int tile, int nOwn, Numbering& faces, Numbering& cells, Tiles& out) {
     const long n = m.nIC;
     const size_t c0 = (size_t)tile * TILE_CELLS, f0 = (size_t)tile * TILE_FACES;
     int* halo = out.halo.data() + (size_t)tile * TILE_HALO;
-    std::fill(std::copy(t.halo.begin(), t.halo.end(), halo), halo + TILE_HALO, (int)c0);
     int* id = out.faceId.data() + f0;
     unsigned* word = out.face.data() + f0;
-    int k = 0;
-    for (const std::vector<int>* g : {&t.inter, &t.pair, &t.ghost})
-        for (int f : *g) id[k++] = f;
-    for (; k < TILE_FACES; k++) id[k] = id[0];
-    const int nInt = (int)t.inter.size(), nPair = (int)t.pair.size();
-    auto face_of = [&](int f) {
-        int i = index_in(t.inter, f);
-        if (i >= 0) return i;
-        i = index_in(t.pair, f);
-        if (i >= 0) return nInt + i;
-        return nInt + nPair + (int)(std::find(t.ghost.begin(), t.ghost.end(), f) - t.ghost.begin());
-    };
     const int* own = out.toUser.data() + c0;
+    int face[TILE_CELLS][6], other[TILE_CELLS][6], ghost[TILE_FACES];
+    int nFace = 0, nHalo = 0, nGhost = 0;
+    bool pairs = false;
+    faces.clear();
+    cells.clear();
+    for (int j = 0; j < 6; j++)
+        for (int i = 0; i < nOwn; i++) {
+            face[i][j] = m.sFace[j * n + own[i]];
+            other[i][j] = m.sOther[j * n + own[i]];
+        }
+    for (int i = 0; i < nOwn; i++)
+        for (int j = 0; j < 6; j++) {
+            const int f = face[i][j], o = other[i][j];
+            if (o < 0) {
+                ghost[nGhost++] = f;
+                continue;
+            }
+            if (faces.add(f, nFace)) id[nFace++] = f;
+            pairs = pairs || f >= m.nIF;
+            const int p = out.toTile[o];
+            if (p / TILE_CELLS != tile && cells.add(p, 0)) halo[nHalo++] = p;
+        }
+    std::sort(halo, halo + nHalo);
+    for (int k = 0; k < nHalo; k++) cells.value[cells.find(halo[k]) - cells.key] = TILE_CELLS + k;
+    if (pairs)
+        for (int i = 0; i < nOwn; i++)
+            for (int j = 0; j < 6; j++) {
+                const int g = m.sPair[j * n + own[i]];
+                if (g >= 0 && faces.add(g, nFace)) id[nFace++] = g;
+            }
+    std::sort(ghost, ghost + nGhost, [&](int a, int b) {
+        return m.fKind[a] != m.fKind[b] ? m.fKind[a] < m.fKind[b] : a < b;
+    });
+    for (int k = 0; k < nGhost; k++)
+        if (faces.add(ghost[k], nFace)) id[nFace++] = ghost[k];
+    std::fill(id + nFace, id + TILE_FACES, id[0]);
+    std::fill(halo + nHalo, halo + TILE_HALO, (int)c0);
     for (int i = 0; i < nOwn; i++) {
         uint64_t sl = 0, pr = 0, nb = 0;
         for (int j = 0; j < 6; j++) {
             const long s = j * n + own[i];
-            const int f = m.sFace[s], o = m.sOther[s], g = m.sPair[s];
+            const int f = face[i][j], o = other[i][j];
             const bool isOwn = m.sFlags[s] & 1;
-            const int lf = face_of(f);
+            const int lf = faces.at(f);
             unsigned lo = 0;
             if (o >= 0) {
                 const int p = out.toTile[o];
-                lo = p / TILE_CELLS == tile ? p % TILE_CELLS : TILE_CELLS + index_in(t.halo, p);
+                lo = p / TILE_CELLS == tile ? p % TILE_CELLS : cells.at(p);
             } else {
                 nb |= 1ull << (TILE_BITS0 + j);
                 if (m.fKind[f] & m.copyBit) nb |= 1ull << (TILE_BITS1 + j);
@@ -302,8 +361,9 @@ inline void fill_tile(const TileMesh& m, int tile, int nOwn, const TileLists& t,
             if (isOwn) sl |= 1ull << (TILE_BITS0 + j);
             word[lf] = (isOwn ? (unsigned)i | lo << 8 : lo | (unsigned)i << 8) | (unsigned)m.fKind[f] << 16 |
                        (f < m.nIF ? TILE_FACE_INTERNAL : 0u);
+            const int g = f >= m.nIF ? m.sPair[s] : -1;
             if (g >= 0) {
-                const int lg = face_of(g);
+                const int lg = faces.at(g);
                 sl |= 1ull << (TILE_BITS1 + j);
                 pr |= (uint64_t)lg << (8 * j);
                 word[lg] = lo | (unsigned)i << 8 | (unsigned)m.fKind[g] << 16;
@@ -315,38 +375,13 @@ inline void fill_tile(const TileMesh& m, int tile, int nOwn, const TileLists& t,
     }
 }
 
-// f(a, b) over the parts of [0, n) on up to 8 host threads; a part whose
-// thread cannot be started runs on this one, and the first exception of any
-// part is rethrown here when all have ended.
-template <typename F> void over_threads(int n, F&& f) {
-    const int nt = std::max(1, std::min({8, (int)std::thread::hardware_concurrency(), n / 256}));
-    std::vector<std::exception_ptr> err(nt);
-    auto part = [&](int k) {
-        try {
-            f((int)((long)n * k / nt), (int)((long)n * (k + 1) / nt));
-        } catch (...) {
-            err[k] = std::current_exception();
-        }
-    };
-    std::vector<std::thread> th;
-    th.reserve(nt);
-    for (int k = 1; k < nt; k++) {
-        try {
-            th.emplace_back(part, k);
-        } catch (const std::system_error&) {
-            part(k);
-        }
-    }
-    part(0);
-    for (auto& x : th) x.join();
-    for (auto& e : err)
-        if (e) std::rethrow_exception(e);
-}
-
 inline void build_tiles(const TileMesh& m, Tiles& t) {
     std::vector<int> cells, start;
-    grow_tiles(m, cells, start);
-    order_tiles(m, cells, start);
+    {
+        const std::vector<int> near = neighbour_list(m);
+        grow_tiles(m, near, cells, start);
+        order_tiles(m, near, cells, start);
+    }
     t.n = (int)start.size() - 1;
     const size_t nPos = (size_t)t.n * TILE_CELLS, nFaces = (size_t)t.n * TILE_FACES;
     if (nFaces > 0x7fffffffu) throw std::length_error("mesh too large for 32-bit tile lists");
@@ -365,12 +400,9 @@ inline void build_tiles(const TileMesh& m, Tiles& t) {
     t.slots.assign(nPos, 0);
     t.pairs.assign(nPos, 0);
     t.nbr.assign(nPos, 0);
-    over_threads(t.n, [&](int a, int b) {
-        TileLists w;
-        for (int k = a; k < b; k++) {
-            list_tile(m, t, k, start[k + 1] - start[k], w);
-            fill_tile(m, k, start[k + 1] - start[k], w, t);
-        }
+    over_threads(t.n, [&](int a, int b, int) {
+        Numbering faces, cells;
+        for (int k = a; k < b; k++) fill_tile(m, k, start[k + 1] - start[k], faces, cells, t);
     });
 }
 
