@@ -234,9 +234,9 @@ __global__ void __launch_bounds__(BLOCK) ghost_kernel(DMesh<T> m, Phys<T> ph, co
     for (int i = 0; i < 5; i++) ghost[i * nBF + b] = out[i];
 }
 
-// Block reduction of one double per thread into out[blockIdx.x]; op 0 sum, 1 max.
+// Block reduction of one double per thread, in thread 0; op 0 sum, 1 max.
 template <int OP, int BS = BLOCK>
-__device__ void block_reduce_store(double v, double* out) {
+__device__ double block_reduce(double v) {
     __shared__ double sh[BS];
     sh[threadIdx.x] = v;
     __syncthreads();
@@ -247,7 +247,13 @@ __device__ void block_reduce_store(double v, double* out) {
         }
         __syncthreads();
     }
-    if (threadIdx.x == 0) out[blockIdx.x] = sh[0];
+    return sh[0];
+}
+
+template <int OP, int BS = BLOCK>
+__device__ void block_reduce_store(double v, double* out) {
+    v = block_reduce<OP, BS>(v);
+    if (threadIdx.x == 0) out[blockIdx.x] = v;
 }
 
 // A thread's share of n partials, those at its index and every THREADS-th after
@@ -277,6 +283,24 @@ __global__ void __launch_bounds__(FINAL_THREADS<OP>) finalize_kernel(const doubl
     block_reduce_store<OP, FINAL_THREADS<OP>>(fold_partials<OP, FINAL_THREADS<OP>>(partials, n), out);
 }
 
+// A step's objective (the sum of nSum values, folded as finalize_kernel folds
+// them) and time step limit (the largest of nMax) in one launch, a block each.
+__global__ void __launch_bounds__(1024) finalize_step_kernel(const double* __restrict__ sums, int nSum, double* sum,
+                                                             const double* __restrict__ largest, int nMax,
+                                                             double* max) {
+    const bool first = blockIdx.x == 0;
+    const double v = first ? block_reduce<0, 1024>(threadIdx.x < BLOCK ? fold_partials<0, BLOCK>(sums, nSum) : 0.0)
+                           : block_reduce<1, 1024>(fold_partials<1, 1024>(largest, nMax));
+    if (threadIdx.x == 0) *(first ? sum : max) = v;
+}
+
+// Kinetic energy 0.5*rho*|U|^2*V of a cell of state q.
+template <typename T> __device__ __forceinline__ T kinetic_energy(const T* q, T V) {
+    T rho = q[0];
+    T Ux = q[1] / rho, Uy = q[2] / rho, Uz = q[3] / rho;
+    return T(0.5) * rho * (Ux * Ux + Uy * Uy + Uz * Uz) * V;
+}
+
 #include "tile_kernels.inc"
 
 // Objective partial sums (FP64): kinetic energy 0.5*rho*|U|^2*V per cell.
@@ -286,12 +310,17 @@ __global__ void __launch_bounds__(BLOCK) ke_kernel(DMesh<T> m, const T* __restri
     const long nIC = m.nIC;
     double v = 0.0;
     if (c < m.nIC) {
-        T rho = u[c];
-        T Ux = u[nIC + c] / rho, Uy = u[2 * nIC + c] / rho, Uz = u[3 * nIC + c] / rho;
-        T ke = T(0.5) * rho * (Ux * Ux + Uy * Uy + Uz * Uz) * m.vol[c];
-        v = (double)ke;
+        const T q[4] = {u[c], u[nIC + c], u[2 * nIC + c], u[3 * nIC + c]};
+        v = (double)kinetic_energy(q, m.vol[c]);
     }
     block_reduce_store<0>(v, partial);
+}
+
+// The same from the cells' kinetic energies.
+template <typename T>
+__global__ void __launch_bounds__(BLOCK) ke_sum_kernel(long nIC, const T* __restrict__ ke, double* partial) {
+    const long c = (long)blockIdx.x * BLOCK + threadIdx.x;
+    block_reduce_store<0>(c < nIC ? (double)ke[c] : 0.0, partial);
 }
 
 // Kinetic energy per cell segment (an ensemble of meshes in one context):
@@ -538,7 +567,7 @@ struct adfvm_ctx {
     void* adjU = nullptr;      // [nIC][5] adjoint between the stages
     void* adjAcc = nullptr;    // [nIC][5] adjoint of u0 accumulated over the stages
     void* adjG = nullptr;      // [nIC][AREC] cell adjoint records
-    double* partial = nullptr; int nPartial = 0;
+    double* partial = nullptr; int nPartial = 0;     // [2][nPartial]: block sums; a step's objective
     double tuneMs[6] = {-1, -1, -1, -1, -1, -1};   // measured time of each stencil kernel (adfvm_autotune)
     // cell segments (adfvm_set_segments): objective per segment
     int nSeg = 1, nSegBlocks = 0;
@@ -834,14 +863,15 @@ struct Stage {
 // residual.
 template <typename T, int MODE>
 void launch_flux_and_stage(adfvm_ctx* c, const T* rec, const T* u, const T* u0, const Stage& st, double dt,
-                           const T* S, T* next, T* rows, T* dtcCell, double* dtcPartial, hipStream_t s) {
+                           const T* S, T* next, T* rows, T* dtcCell, double* dtcPartial, hipStream_t s,
+                           T* keCell = nullptr) {
     KTimer kt(c, MODE == 0 ? "flux_stage_kernel" : "residual_kernel", s);
     with_stream(c->stream, [&](auto SP) {
         with_ghosts(c->hasGhostKernel, [&](auto G) {
             constexpr bool ST = decltype(SP)::value, GH = decltype(G)::value;
             flux_stage_kernel<T, MODE, ST, GH><<<c->nTiles, TILE_THREADS, 0, s>>>(
                 dmesh<T>(c), dtiles<T>(c), phys_cast<T>(c->phd), rec, u, u0, (T)st.ai, (T)(-st.beta), (T)dt, S, next,
-                rows, dtcCell, dtcPartial);
+                rows, dtcCell, dtcPartial, keCell);
         });
     });
 }
@@ -862,13 +892,14 @@ void launch_flux_and_stage(adfvm_ctx* c, const T* rec, const T* u, const T* u0, 
 // and where the rows written are those read.
 template <typename T, int MODE>
 void launch_stage(adfvm_ctx* c, const T* u, bool user, T* copy, T* rec, T* work, const T* u0, const Stage& st, double dt,
-                  const T* S, T* next, T* rows, T* dtcCell, double* dtcPartial, hipStream_t s) {
+                  const T* S, T* next, T* rows, T* dtcCell, double* dtcPartial, hipStream_t s,
+                  T* keCell = nullptr) {
     auto over_u = [&](const T* out, long n) { return user && out && out < u + 5L * c->nIC && u < out + n; };
     const bool overlap = over_u(rows, 5L * c->nIC) || over_u(dtcCell, c->nIC);
     if (!c->tileRing || overlap || (rec && c->nTiles > one_launch_rec_tiles(c))) {
         T* r = rec ? rec : work;
         launch_grad<T>(c, u, user, copy, r, s);
-        launch_flux_and_stage<T, MODE>(c, r, user ? copy : u, u0, st, dt, S, next, rows, dtcCell, dtcPartial, s);
+        launch_flux_and_stage<T, MODE>(c, r, user ? copy : u, u0, st, dt, S, next, rows, dtcCell, dtcPartial, s, keCell);
         return;
     }
     KTimer kt(c, MODE == 0 ? "tile_stage_kernel" : "tile_residual_kernel", s);
@@ -877,7 +908,7 @@ void launch_stage(adfvm_ctx* c, const T* u, bool user, T* copy, T* rec, T* work,
             constexpr bool ST = decltype(SP)::value, GH = decltype(G)::value;
             tile_stage_kernel<T, MODE, ST, GH><<<c->nTiles, TILE_THREADS, 0, s>>>(
                 dmesh<T>(c), dtiles<T>(c), phys_cast<T>(c->phd), u, user, copy, rec, u0, (T)st.ai, (T)(-st.beta), (T)dt, S,
-                next, rows, dtcCell, dtcPartial);
+                next, rows, dtcCell, dtcPartial, keCell);
         });
     });
 }
@@ -941,10 +972,17 @@ int primal_step_t(adfvm_ctx* c, T* u, double dt, const T* S, double* dtc_out, do
     if (tape) tape_slots(c, ns, tape, rec);
     const int objStage = objective_stage(c, ns);
     const int dtcStage = ns > 1 ? 1 : 0;    // density.py:412-413
+    // the cells' kinetic energies at the first intermediate stage come from the
+    // kernel that makes it: five rows less to write, scattered by the caller's
+    // numbering, and to read again (128^3 FP32 step without a tape 1005 -> 940 us)
+    const bool ke1 = obj_out && objStage == 1 && c->objective == ADFVM_OBJ_KINETIC_ENERGY && c->nSeg <= 1;
+    T* keCell = ke1 ? P<T>(c->rows1) : nullptr;
+    double* kePartial = c->partial + c->nPartial;
+    const int gKe = grid_for(c->nIC);
     // the objective stage's state in the caller's numbering, where one is needed
-    T* rows1 = ns == 1 ? nullptr : tape ? tape : (obj_out && objStage == 1) ? P<T>(c->rows1) : nullptr;
+    T* rows1 = ns == 1 ? nullptr : tape ? tape : (obj_out && objStage == 1 && !ke1) ? P<T>(c->rows1) : nullptr;
     for (int i = 0; i < ns; i++) {
-        if (i == objStage && obj_out) launch_objective<T>(c, i == 0 ? u : rows1, obj_out, s);
+        if (i == objStage && obj_out && !ke1) launch_objective<T>(c, i == 0 ? u : rows1, obj_out, s);
         const bool wantDtc = (i == dtcStage) && dtc_out;
         const T* u0 = (i > 0 && st[i].a0 != 0.0) ? P<T>(c->st[0]) : nullptr;
         // the last stage writes the caller's state in place: the kernels of
@@ -952,8 +990,19 @@ int primal_step_t(adfvm_ctx* c, T* u, double dt, const T* S, double* dtc_out, do
         const bool last = i == ns - 1;
         launch_stage<T, 0>(c, i == 0 ? u : P<T>(c->st[i]), i == 0, i == 0 ? P<T>(c->st[0]) : nullptr,
                            tape ? rec[i] : nullptr, P<T>(c->rec[i]), u0, st[i], dt, S, last ? nullptr : P<T>(c->st[i + 1]),
-                           last ? u : i == 0 ? rows1 : nullptr, nullptr, wantDtc ? c->partial : nullptr, s);
-        if (wantDtc) finalize_kernel<1><<<1, FINAL_THREADS<1>, 0, s>>>(c->partial, c->nTiles, dtc_out);
+                           last ? u : i == 0 ? rows1 : nullptr, nullptr, wantDtc ? c->partial : nullptr, s,
+                           i == 0 ? keCell : nullptr);
+        if (i != dtcStage) continue;
+        if (ke1) {
+            KTimer kt(c, "objective", s);
+            ke_sum_kernel<T><<<gKe, BLOCK, 0, s>>>(c->nIC, keCell, kePartial);
+            if (wantDtc)
+                finalize_step_kernel<<<2, 1024, 0, s>>>(kePartial, gKe, obj_out, c->partial, c->nTiles, dtc_out);
+            else
+                finalize_kernel<0><<<1, FINAL_THREADS<0>, 0, s>>>(kePartial, gKe, obj_out);
+        } else if (wantDtc) {
+            finalize_kernel<1><<<1, FINAL_THREADS<1>, 0, s>>>(c->partial, c->nTiles, dtc_out);
+        }
     }
     HIPCHK(c, hipGetLastError());
     return ADFVM_OK;
@@ -1128,7 +1177,7 @@ extern "C" int adfvm_ctx_create(const adfvm_solver_desc* d, const adfvm_physics*
     if ((rc = upload(c, (void**)&c->patches, c->hpatches)) != ADFVM_OK) return rc;
     c->stream = stream_auto(c);
     c->nPartial = std::max(grid_bs(std::max<long>(nIC, nF), kBlockChoices[0]) + 1, c->nTiles);   // the smallest block size
-    HIPCHK(c, hipMalloc((void**)&c->partial, c->nPartial * sizeof(double)));
+    HIPCHK(c, hipMalloc((void**)&c->partial, 2L * c->nPartial * sizeof(double)));
     HIPCHK(c, hipMalloc((void**)&c->scal, 16 * sizeof(double)));
     return ADFVM_OK;
 }
