@@ -913,6 +913,25 @@ void launch_stage(adfvm_ctx* c, const T* u, bool user, T* copy, T* rec, T* work,
     });
 }
 
+// Whether steps turn the caller's rows into records, and back, in launches of
+// their own.  In the tile kernels a tile's cells lie in runs of 3 to 6 in a row,
+// of which every line is read or written by several tiles, apart in time: at
+// 128^3 FP32 a step's first and last stages took 160 us longer than with records,
+// the conversions take 27 each.  A step 940 -> 816 us, with its adjoint step
+// 2185 -> 1962; 64^3 (4.2k tiles) 120.5 -> 115 and 279 -> 277, 72^3 382 -> 369; 48^3
+// (1.8k tiles) 155 -> 157, cells of an O-grid (longer runs) 131k (2.2k tiles) 193
+// -> 202, 410k (6.9k tiles) 439 -> 443.  12 tiles a compute unit:
+constexpr int CONVERT_TILES = 3072;
+bool converts_rows(const adfvm_ctx* c) { return c->nTiles > CONVERT_TILES; }
+template <typename T> void launch_to_records(adfvm_ctx* c, const T* rows, T* rec, hipStream_t s) {
+    KTimer kt(c, "to_records_kernel", s);
+    to_records_kernel<T><<<grid_for(c->nIC), BLOCK, 0, s>>>(c->nIC, c->toTile, rows, rec);
+}
+template <typename T> void launch_to_rows(adfvm_ctx* c, const T* rec, T* rows, hipStream_t s) {
+    KTimer kt(c, "to_rows_kernel", s);
+    to_rows_kernel<T><<<grid_for(c->nIC), BLOCK, 0, s>>>(c->nIC, c->toTile, rec, rows);
+}
+
 template <typename T> void launch_objective(adfvm_ctx* c, const T* u, double* out, hipStream_t s) {
     KTimer kt(c, "objective", s);
     if (c->objective == ADFVM_OBJ_KINETIC_ENERGY && c->nSeg > 1) {
@@ -981,17 +1000,22 @@ int primal_step_t(adfvm_ctx* c, T* u, double dt, const T* S, double* dtc_out, do
     const int gKe = grid_for(c->nIC);
     // the objective stage's state in the caller's numbering, where one is needed
     T* rows1 = ns == 1 ? nullptr : tape ? tape : (obj_out && objStage == 1 && !ke1) ? P<T>(c->rows1) : nullptr;
+    const bool convert = converts_rows(c);
+    T* const u0rec = P<T>(c->st[0]);
+    if (convert) launch_to_records<T>(c, u, u0rec, s);
     for (int i = 0; i < ns; i++) {
         if (i == objStage && obj_out && !ke1) launch_objective<T>(c, i == 0 ? u : rows1, obj_out, s);
         const bool wantDtc = (i == dtcStage) && dtc_out;
-        const T* u0 = (i > 0 && st[i].a0 != 0.0) ? P<T>(c->st[0]) : nullptr;
+        const T* u0 = (i > 0 && st[i].a0 != 0.0) ? u0rec : nullptr;
         // the last stage writes the caller's state in place: the kernels of
-        // this step read it no more (its records are st[0])
-        const bool last = i == ns - 1;
-        launch_stage<T, 0>(c, i == 0 ? u : P<T>(c->st[i]), i == 0, i == 0 ? P<T>(c->st[0]) : nullptr,
-                           tape ? rec[i] : nullptr, P<T>(c->rec[i]), u0, st[i], dt, S, last ? nullptr : P<T>(c->st[i + 1]),
-                           last ? u : i == 0 ? rows1 : nullptr, nullptr, wantDtc ? c->partial : nullptr, s,
-                           i == 0 ? keCell : nullptr);
+        // this step read it no more (its records are st[0]); st[1] is free then
+        const bool last = i == ns - 1, user = i == 0 && !convert;
+        T* rows = last ? u : i == 0 ? rows1 : nullptr;
+        T* next = !last ? P<T>(c->st[i + 1]) : convert ? P<T>(c->st[1]) : nullptr;
+        launch_stage<T, 0>(c, user ? u : P<T>(c->st[i]), user, user ? u0rec : nullptr, tape ? rec[i] : nullptr,
+                           P<T>(c->rec[i]), u0, st[i], dt, S, next, convert ? nullptr : rows, nullptr,
+                           wantDtc ? c->partial : nullptr, s, i == 0 ? keCell : nullptr);
+        if (convert && rows) launch_to_rows<T>(c, next, rows, s);
         if (i != dtcStage) continue;
         if (ke1) {
             KTimer kt(c, "objective", s);
