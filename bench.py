@@ -52,6 +52,8 @@ def kernel_bytes(name, s, nC, nF, nG, nO=None):
         return nC * (20 + 5 + 1 + 20) * s + nF * 16 * s + 4 * nF + 24 * nC
     if name == 'grad_vjp_kernel':      # w, cell adjoint records, ubar, acc (2 of 3), slot geometry -> ubar, acc
         return nC * (5 + 20 + 5 + 10. / 3 + 24 + 5 + 10. / 3) * s + 24 * nC
+    if name in ('to_records_kernel', 'to_rows_kernel'):      # five rows <-> records, positions
+        return nC * (10 * s + 4)
     recs = 2 * nF if nO is None else (nF - nG) + nO + 2 * nG
     idx = 8 * nF if nO is None else 4 * (nF - nG) + 8 * nG
     if name == 'face_vjp_kernel':      # u, grad, ubar, V, 16 face rows -> face adjoint records
