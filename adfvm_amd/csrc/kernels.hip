@@ -847,7 +847,7 @@ template <typename T> void launch_grad(adfvm_ctx* c, const T* u, bool user, T* c
 }
 
 // u_{i+1} = a0*u0 + ai*u_i - beta*(L-S)*dt.  Every stage of the tables
-// below with a0 != 0 has a0 + ai = 1, and stage_kernel evaluates it as
+// below with a0 != 0 has a0 + ai = 1, and the stage kernels evaluate it as
 // u0 + (ai*(u_i - u0) - beta*(L-S)*dt), so sum(V*u) is kept up to unbiased
 // rounding.  (Taken as a0*u0 + ai*u_i with the coefficients rounded apart,
 // SSP-RK3's 1/3 and 2/3 both round up in FP32, to a sum of 1 + 2^-25: the
