@@ -234,17 +234,21 @@ __global__ void __launch_bounds__(BLOCK) ghost_kernel(DMesh<T> m, Phys<T> ph, co
     for (int i = 0; i < 5; i++) ghost[i * nBF + b] = out[i];
 }
 
-// Block reduction of one double per thread, in thread 0; op 0 sum, 1 max.
+// What the reductions combine two values by: op 0 their sum, 1 the larger of
+// them.  A NaN on either side is kept: a comparison alone would drop the one on
+// its left, and the time step limit of a diverged state would look finite.
+template <int OP> __device__ __forceinline__ double combine(double a, double b) {
+    return OP == 0 ? a + b : (a > b || a != a ? a : b);
+}
+
+// Block reduction of one double per thread, in thread 0.
 template <int OP, int BS = BLOCK>
 __device__ double block_reduce(double v) {
     __shared__ double sh[BS];
     sh[threadIdx.x] = v;
     __syncthreads();
     for (int s = BS / 2; s > 0; s >>= 1) {
-        if (threadIdx.x < s) {
-            double a = sh[threadIdx.x], b = sh[threadIdx.x + s];
-            sh[threadIdx.x] = OP == 0 ? a + b : (a > b ? a : b);
-        }
+        if (threadIdx.x < s) sh[threadIdx.x] = combine<OP>(sh[threadIdx.x], sh[threadIdx.x + s]);
         __syncthreads();
     }
     return sh[0];
@@ -269,7 +273,7 @@ __device__ __forceinline__ double fold_partials(const double* __restrict__ parti
 #pragma unroll
         for (int k = 0; k < BATCH; k++) x[k] = i + k * THREADS < n ? partials[i + k * THREADS] : none;
 #pragma unroll
-        for (int k = 0; k < BATCH; k++) v = OP == 0 ? v + x[k] : (v > x[k] ? v : x[k]);
+        for (int k = 0; k < BATCH; k++) v = combine<OP>(v, x[k]);
     }
     return v;
 }

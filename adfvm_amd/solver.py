@@ -146,7 +146,10 @@ class Solver(object):
             if isinstance(dts, np.ndarray):
                 dt = float(dts[timeIndex]) if timeIndex < len(dts) else dt
             elif not fixed:
-                dt = min(2 * self.CFL / dtc.item(), dt * self.stepFactor, endTime - t)
+                limit = dtc.item()
+                if limit != limit:       # no next dt: min() below would return NaN and end the loop silently
+                    raise FloatingPointError('NaN in the time step limit at step %d (t=%g)' % (timeIndex, t))
+                dt = min(2 * self.CFL / limit, dt * self.stepFactor, endTime - t)
             if write and mode != 'forward':
                 if mode in ('orig', 'simulation'):
                     self.writeFields(t)

@@ -1,0 +1,50 @@
+"""A state that holds a NaN gives a NaN time step limit, whatever the mesh's
+size and wherever the NaN is."""
+import numpy as np
+import pytest
+
+from adfvm_amd import config, meshgen
+from tests import casefactory as cf
+
+MESHES = {
+    'part_of_a_tile': lambda: meshgen.periodic_box((3, 3, 3)),
+    'tiles_and_a_part': lambda: meshgen.permute_and_rcm(meshgen.periodic_box((13, 11, 9)), seed=3),
+    'tube': lambda: meshgen.shock_tube(131),
+    'above_1024_tiles': lambda: meshgen.permute_and_rcm(meshgen.periodic_box((41, 42, 43)), seed=3),
+}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('name', sorted(MESHES))
+@pytest.mark.parametrize('prec', [np.float32, np.float64])
+@pytest.mark.parametrize('where', ['all', 'first', 'middle', 'last'])
+@pytest.mark.parametrize('objective', [None, ('kinetic_energy',)])
+def test_limit_of_a_state_with_a_nan(name, prec, where, objective):
+    """Every cell, or one cell, of 27 to 74046."""
+    import torch
+    case = cf.CaseDef(MESHES[name](), {}, 1e-3, objective=objective)
+    ctx = case.context(prec)
+    u = torch.as_tensor(cf.smooth_state(case, 4).astype(prec), device='cuda').contiguous()
+    n = ctx.nIC
+    u[:, {'all': slice(None), 'first': 0, 'middle': n // 2, 'last': n - 1}[where]] = float('nan')
+    dtc = torch.zeros(1, dtype=torch.float64, device='cuda')
+    obj = torch.zeros(1, dtype=torch.float64, device='cuda')
+    ctx.primal_step(u, 1e-6, dtc_out=dtc, obj_out=obj)
+    assert torch.isnan(dtc).all()
+    if objective:
+        assert torch.isnan(obj).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('n', [5, 41])
+def test_run_with_time_step_control_stops(n):
+    """A run whose limit is NaN has no next time step: it stops with the
+    error of its NaN report, which here is not due."""
+    case, params = cf.tgv(n)
+    u = cf.tgv_state(case, params)
+    u[4, 3] = np.nan
+    precision = config.precision
+    s = cf.rcf(case, u, np.float64, CFL=0.5, stepFactor=1.2)
+    with pytest.raises(FloatingPointError):
+        s.run(endTime=1.0, dt=1e-6, nSteps=5, reportInterval=1000, mode='forward')
+    config.set_precision(precision)
