@@ -558,9 +558,11 @@ struct adfvm_ctx {
     int* nbFull = nullptr;       // ghost-extended neighbour [nF]
     void* ghost = nullptr;
     // adjoint viscosity, from its first call on: [6][nIC] slot coefficients,
-    // [nIC] diagonal, [nIC] eigenvalue; the patches' tables (sweeps at a time,
-    // patches) and [nPos][12] slot coefficients, diagonal, right side
+    // [nIC] diagonal, [nIC] eigenvalue; from its first call outside a capture on,
+    // where they pay, the patches' tables (sweeps at a time, patches) and [nPos][12]
+    // slot coefficients, diagonal, right side
     void* visc = nullptr;
+    bool ringsTried = false;
     int ringK = 1, ringN = 0;
     RingCell* ringCell = nullptr;
     int* ringCount = nullptr;

@@ -315,7 +315,11 @@ int adfvm_set_mesh_grad(adfvm_ctx* ctx, void* mesh_grad);
  * `iterations` Jacobi sweeps of the implicit step
  * (1 + dt/V sum_f A DT_f/delta_f) phi - dt/V sum_f (A DT_f/delta_f) phi_nb = ua/V
  * over internal faces (the reference runs 1000), then ua = phi V in place.
- * m2norm_out (device [nIC], nullable): the scaled viscosity per cell. */
+ * m2norm_out (device [nIC], nullable): the scaled viscosity per cell.
+ * A context's first call allocates device memory, and its first call outside a
+ * stream capture makes the tables for several sweeps a launch (more memory, one
+ * synchronisation of the stream).  Until then it sweeps one at a time; results
+ * are the same. */
 #define ADFVM_VISC_UNIFORM 0
 #define ADFVM_VISC_ABARBANEL 1
 #define ADFVM_VISC_TURKEL 2
