@@ -19,6 +19,9 @@
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
+#include <exception>
+#include <future>
+#include <initializer_list>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -550,7 +553,8 @@ struct adfvm_ctx {
     std::string err;
     std::vector<DPatch> hpatches;
     std::vector<int> hBPatch;  // boundary face -> patch (host copy)
-    // device
+    // device; the tables are parts of faceTables, meshTables and tileTables
+    void *faceTables = nullptr, *meshTables = nullptr, *tileTables = nullptr;
     void* geo = nullptr; void* vol = nullptr; void* bcval = nullptr;
     int* sFace = nullptr; int* sOther = nullptr; unsigned char* sFlags = nullptr; int* sPair = nullptr;
     int* owner = nullptr; int* bPatch = nullptr; DPatch* patches = nullptr;
@@ -577,6 +581,7 @@ struct adfvm_ctx {
     double tuneMs[6] = {-1, -1, -1, -1, -1, -1};   // measured time of each stencil kernel (adfvm_autotune)
     // cell segments (adfvm_set_segments): objective per segment
     int nSeg = 1, nSegBlocks = 0;
+    void* segTables = nullptr;  // the three below
     long* segCell = nullptr; int* segBlock = nullptr; int* blockSeg = nullptr;
     double* scal = nullptr;    // small device scalars
     int* fOther = nullptr; unsigned char* fKind = nullptr;
@@ -709,92 +714,64 @@ template <typename T> DTiles<T> dtiles(const adfvm_ctx* c) {
 constexpr int ONE_LAUNCH_TILES = 5120;
 int one_launch_rec_tiles(const adfvm_ctx* c) { return c->prec == 8 && c->hasGhostKernel ? 256 : 1024; }
 
-template <typename T> int upload(adfvm_ctx* ctx, void** dst, const std::vector<T>& v) {
-    HIPCHK(ctx, hipMalloc(dst, std::max<size_t>(1, v.size()) * sizeof(T)));
-    if (!v.empty()) HIPCHK(ctx, hipMemcpy(*dst, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
+// Host tables that go to the device together, into parts of one allocation.  A
+// copy takes 10 us and more whatever its size, so the small ones go as one, from a
+// host buffer (a 1000-cell tube's context 0.71 -> 0.35 ms).
+struct Table {
+    void** part;
+    const void* host;
+    size_t bytes;
+};
+template <typename D, typename T, typename A> Table table(D*& part, const std::vector<T, A>& v) {
+    return {(void**)&part, v.data(), v.size() * sizeof(T)};
+}
+int upload(adfvm_ctx* ctx, void** base, std::initializer_list<Table> tables) {
+    constexpr size_t ALIGN = 256, SMALL = 128 << 10;
+    auto padded = [](size_t bytes) { return (bytes + ALIGN - 1) / ALIGN * ALIGN; };
+    size_t all = ALIGN, small = 0, at = 0;
+    for (const Table& t : tables) {
+        all += padded(t.bytes);
+        if (t.bytes <= SMALL) small += padded(t.bytes);
+    }
+    HIPCHK(ctx, hipMalloc(base, all));
+    Buffer<char> host(small);
+    for (const Table& t : tables) {
+        if (t.bytes > SMALL) continue;
+        *t.part = (char*)*base + at;
+        if (t.bytes) std::memcpy(host.data() + at, t.host, t.bytes);
+        at += padded(t.bytes);
+    }
+    if (small) HIPCHK(ctx, hipMemcpy(*base, host.data(), small, hipMemcpyHostToDevice));
+    for (const Table& t : tables) {
+        if (t.bytes <= SMALL) continue;
+        *t.part = (char*)*base + at;
+        HIPCHK(ctx, hipMemcpy(*t.part, t.host, t.bytes, hipMemcpyHostToDevice));
+        at += padded(t.bytes);
+    }
     return ADFVM_OK;
 }
 
-template <typename T> int create_typed(adfvm_ctx* ctx, const adfvm_solver_desc* d, const Tiles& t) {
-    const std::vector<int>& toUser = t.toUser;
-    const long nF = ctx->nF, nIC = ctx->nIC, nBF = ctx->nBF;
-    std::vector<T> geo((size_t)G_ROWS * nF);
-    for (long f = 0; f < nF; f++) {
-        geo[G_A * nF + f] = (T)d->areas[f];
-        for (int i = 0; i < 3; i++) geo[(G_NX + i) * nF + f] = (T)d->normals[3 * f + i];
-        geo[G_W * nF + f] = (T)d->weights[f];
-        geo[G_DELTA * nF + f] = (T)d->deltas[f];
-        for (int i = 0; i < 3; i++) geo[(G_DX + i) * nF + f] = (T)d->deltasUnit[3 * f + i];
-        geo[G_LW0 * nF + f] = (T)d->linearWeights[2 * f];
-        geo[G_LW1 * nF + f] = (T)d->linearWeights[2 * f + 1];
-        for (int i = 0; i < 3; i++) {
-            geo[(G_Q0X + i) * nF + f] = (T)d->quadraticWeights[6 * f + i];
-            geo[(G_Q1X + i) * nF + f] = (T)d->quadraticWeights[6 * f + 3 + i];
-        }
-    }
-    int rc;
-    if ((rc = upload(ctx, &ctx->geo, geo)) != ADFVM_OK) return rc;
-    std::vector<T> vol(nIC);
-    for (long c = 0; c < nIC; c++) vol[c] = (T)d->volumes[c];
-    if ((rc = upload(ctx, &ctx->vol, vol)) != ADFVM_OK) return rc;
-    const long nPos = ctx->nPos();
-    // Gauss-gradient geometry per cell slot, by position, computed in FP64 and cast once:
-    // the cell's outward S*n and the weight w' of the other side's value
-    // (phi_f = phi_c (1 - w') + phi_other w'), streamed by the gradient
-    // kernels instead of gathering face rows.
-    std::vector<T> sn((size_t)24 * nPos, T(0)), tvol(nPos, T(1));
-    over_threads((int)(nPos / TILE_CELLS), [&](int a, int b, int) {
-        for (long p = (long)a * TILE_CELLS; p < (long)b * TILE_CELLS; p++) {
-            const long c = toUser[p];
-            if (c < 0) continue;
-            tvol[p] = (T)d->volumes[c];
-            for (int j = 0; j < 6; j++) {
-                const long f = d->cellFaces[6 * c + j];
-                const bool own = d->cellOwner[6 * c + j] != 0;
-                const double sgn = own ? 1.0 : -1.0;
-                const double w = d->weights[f];
-                for (int k = 0; k < 3; k++) sn[24 * p + 4 * j + k] = (T)(sgn * (d->areas[f] * d->normals[3 * f + k]));
-                sn[24 * p + 4 * j + 3] = (T)(own ? 1.0 - w : w);
+// The tables by face and by patch.
+template <typename T> int create_face_tables(adfvm_ctx* ctx, const adfvm_solver_desc* d) {
+    const long nF = ctx->nF, nIC = ctx->nIC;
+    Buffer<T> geo((size_t)G_ROWS * nF);
+    over_threads((int)nF, 2 * CELL_GRAIN, [&](int a, int b, int) {
+        for (long f = a; f < b; f++) {
+            geo[G_A * nF + f] = (T)d->areas[f];
+            for (int i = 0; i < 3; i++) geo[(G_NX + i) * nF + f] = (T)d->normals[3 * f + i];
+            geo[G_W * nF + f] = (T)d->weights[f];
+            geo[G_DELTA * nF + f] = (T)d->deltas[f];
+            for (int i = 0; i < 3; i++) geo[(G_DX + i) * nF + f] = (T)d->deltasUnit[3 * f + i];
+            geo[G_LW0 * nF + f] = (T)d->linearWeights[2 * f];
+            geo[G_LW1 * nF + f] = (T)d->linearWeights[2 * f + 1];
+            for (int i = 0; i < 3; i++) {
+                geo[(G_Q0X + i) * nF + f] = (T)d->quadraticWeights[6 * f + i];
+                geo[(G_Q1X + i) * nF + f] = (T)d->quadraticWeights[6 * f + 3 + i];
             }
         }
     });
-    {
-        // the tables the blocks are filled from, freed at the end of the scope
-        struct Temp {
-            void* p[7] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
-            ~Temp() { for (void* q : p) if (q) (void)hipFree(q); }
-        } tmp;
-        if ((rc = upload(ctx, &tmp.p[0], sn)) != ADFVM_OK) return rc;
-        if ((rc = upload(ctx, &tmp.p[1], tvol)) != ADFVM_OK) return rc;
-        if ((rc = upload(ctx, &tmp.p[2], t.nbr)) != ADFVM_OK) return rc;
-        if ((rc = upload(ctx, &tmp.p[3], t.slots)) != ADFVM_OK) return rc;
-        if ((rc = upload(ctx, &tmp.p[4], t.halo)) != ADFVM_OK) return rc;
-        if ((rc = upload(ctx, &tmp.p[5], t.face)) != ADFVM_OK) return rc;
-        HIPCHK(ctx, hipMalloc((void**)&ctx->tileBlock, (size_t)ctx->nTiles * TileBlock<T>::BYTES));
-        HIPCHK(ctx, hipMalloc(&ctx->tileFaceW, ctx->nTileFaces() * sizeof(T)));
-        tile_block_kernel<T><<<ctx->nTiles, TILE_FACES>>>(
-            (const T*)ctx->geo, nF, (const T*)tmp.p[0], (const unsigned long long*)tmp.p[2],
-            (const unsigned long long*)tmp.p[3], (const int*)tmp.p[4], ctx->toUser, (const T*)tmp.p[1],
-            (const unsigned*)tmp.p[5], ctx->tileFaceId, ctx->tileBlock, (T*)ctx->tileFaceW);
-        HIPCHK(ctx, hipGetLastError());
-        // the rings around the tiles, where stages are to take one launch
-        // (launch_stage): not where one does not fit, or the memory for them is
-        // not to be had
-        if (ctx->nTiles <= ONE_LAUNCH_TILES &&
-            hipMalloc((void**)&ctx->tileRing, (size_t)ctx->nTiles * sizeof(TileRing)) == hipSuccess) {
-            int over = 0;
-            if ((rc = upload(ctx, &tmp.p[6], std::vector<int>(1, 0))) != ADFVM_OK) return rc;
-            tile_ring_kernel<<<ctx->nTiles, TILE_HALO>>>(nIC, (const int*)tmp.p[4], ctx->toUser, ctx->toTile, ctx->sOther,
-                                                         ctx->sFace, ctx->fKind, ctx->tileRing, (int*)tmp.p[6]);
-            HIPCHK(ctx, hipGetLastError());
-            HIPCHK(ctx, hipMemcpy(&over, tmp.p[6], sizeof(int), hipMemcpyDeviceToHost));
-            if (over) { (void)hipFree(ctx->tileRing); ctx->tileRing = nullptr; }
-        } else {
-            (void)hipGetLastError();
-            ctx->tileRing = nullptr;
-        }
-        HIPCHK(ctx, hipDeviceSynchronize());
-    }
+    std::vector<T> vol(nIC);
+    for (long c = 0; c < nIC; c++) vol[c] = (T)d->volumes[c];
     // boundary-condition values
     std::vector<T> vals;
     for (int p = 0; p < d->nPatches; p++) {
@@ -814,7 +791,76 @@ template <typename T> int create_typed(adfvm_ctx* ctx, const adfvm_solver_desc* 
         D.valDir = add(P.direction, 3L * P.nFaces);
         D.hasDir = P.direction != nullptr;
     }
-    if ((rc = upload(ctx, &ctx->bcval, vals)) != ADFVM_OK) return rc;
+    return upload(ctx, &ctx->faceTables,
+                  {table(ctx->geo, geo), table(ctx->vol, vol), table(ctx->bcval, vals), table(ctx->patches, ctx->hpatches)});
+}
+
+// The tables by tile and the work buffers.
+template <typename T> int create_tile_tables(adfvm_ctx* ctx, const adfvm_solver_desc* d, const Tiles& t) {
+    const Buffer<int>& toUser = t.toUser;
+    const long nF = ctx->nF, nIC = ctx->nIC, nBF = ctx->nBF;
+    int rc;
+    if ((rc = upload(ctx, &ctx->tileTables, {table(ctx->toUser, t.toUser), table(ctx->toTile, t.toTile),
+                                             table(ctx->tileFaceId, t.faceId), table(ctx->tilePairs, t.pairs)})) != ADFVM_OK)
+        return rc;
+    const long nPos = ctx->nPos();
+    // Gauss-gradient geometry per cell slot, by position, computed in FP64 and cast once:
+    // the cell's outward S*n and the weight w' of the other side's value
+    // (phi_f = phi_c (1 - w') + phi_other w'), streamed by the gradient
+    // kernels instead of gathering face rows.
+    Buffer<T> sn((size_t)24 * nPos);
+    over_threads(ctx->nTiles, TILE_GRAIN, [&](int a, int b, int) {
+        for (long p = (long)a * TILE_CELLS; p < (long)b * TILE_CELLS; p++) {
+            const long c = toUser[p];
+            if (c < 0) {
+                std::fill_n(&sn[24 * p], 24, T(0));
+                continue;
+            }
+            for (int j = 0; j < 6; j++) {
+                const long f = d->cellFaces[6 * c + j];
+                const bool own = d->cellOwner[6 * c + j] != 0;
+                const double sgn = own ? 1.0 : -1.0;
+                const double w = d->weights[f];
+                for (int k = 0; k < 3; k++) sn[24 * p + 4 * j + k] = (T)(sgn * (d->areas[f] * d->normals[3 * f + k]));
+                sn[24 * p + 4 * j + 3] = (T)(own ? 1.0 - w : w);
+            }
+        }
+    });
+    {
+        // the tables the blocks are filled from, freed at the end of the scope
+        struct Temp {
+            void* p = nullptr;
+            ~Temp() { if (p) (void)hipFree(p); }
+        } tmp;
+        void *dsn, *nbr, *slots, *halo, *face, *over;
+        const std::vector<int> none(1, 0);
+        if ((rc = upload(ctx, &tmp.p, {table(dsn, sn), table(nbr, t.nbr), table(slots, t.slots), table(halo, t.halo),
+                                       table(face, t.face), table(over, none)})) != ADFVM_OK)
+            return rc;
+        HIPCHK(ctx, hipMalloc((void**)&ctx->tileBlock, (size_t)ctx->nTiles * TileBlock<T>::BYTES));
+        HIPCHK(ctx, hipMalloc(&ctx->tileFaceW, ctx->nTileFaces() * sizeof(T)));
+        tile_block_kernel<T><<<ctx->nTiles, TILE_FACES>>>(
+            (const T*)ctx->geo, nF, (const T*)dsn, (const unsigned long long*)nbr, (const unsigned long long*)slots,
+            (const int*)halo, ctx->toUser, (const T*)ctx->vol, (const unsigned*)face, ctx->tileFaceId, ctx->tileBlock,
+            (T*)ctx->tileFaceW);
+        HIPCHK(ctx, hipGetLastError());
+        // the rings around the tiles, where stages are to take one launch
+        // (launch_stage): not where one does not fit, or the memory for them is
+        // not to be had
+        if (ctx->nTiles <= ONE_LAUNCH_TILES &&
+            hipMalloc((void**)&ctx->tileRing, (size_t)ctx->nTiles * sizeof(TileRing)) == hipSuccess) {
+            int unfit = 0;
+            tile_ring_kernel<<<ctx->nTiles, TILE_HALO>>>(nIC, (const int*)halo, ctx->toUser, ctx->toTile, ctx->sOther,
+                                                         ctx->sFace, ctx->fKind, ctx->tileRing, (int*)over);
+            HIPCHK(ctx, hipGetLastError());
+            HIPCHK(ctx, hipMemcpy(&unfit, over, sizeof(int), hipMemcpyDeviceToHost));
+            if (unfit) { (void)hipFree(ctx->tileRing); ctx->tileRing = nullptr; }
+        } else {
+            (void)hipGetLastError();
+            ctx->tileRing = nullptr;
+        }
+        HIPCHK(ctx, hipDeviceSynchronize());
+    }
     // work buffers
     const size_t st = 5 * nIC * sizeof(T), sp = 5 * nPos * sizeof(T);
     HIPCHK(ctx, hipMalloc(&ctx->ghost, std::max<size_t>(1, 5 * nBF) * sizeof(T)));
@@ -1042,12 +1088,10 @@ int primal_step_t(adfvm_ctx* c, T* u, double dt, const T* S, double* dtc_out, do
 
 // ------------------------------------------------------------- C ABI -----
 
-extern "C" int adfvm_ctx_create(const adfvm_solver_desc* d, const adfvm_physics* ph, adfvm_ctx** out) {
-    if (!d || !ph || !out) return ADFVM_ERR_INVALID;
-    *out = nullptr;
-    adfvm_ctx* c = new adfvm_ctx();
+// Checks the mesh and the patches, and makes c's tables and work buffers.
+static int fill_context(adfvm_ctx* c, const adfvm_solver_desc* d, const adfvm_physics* ph) {
     auto bad = [&](const std::string& m) { c->err = m; return ADFVM_ERR_INVALID; };
-    if (ph->precision != 4 && ph->precision != 8) { int r = bad("precision must be 4 or 8"); *out = c; return r; }
+    if (ph->precision != 4 && ph->precision != 8) return bad("precision must be 4 or 8");
     c->prec = ph->precision;
     c->nIC = d->sizes.nInternalCells; c->nIF = d->sizes.nInternalFaces; c->nF = d->sizes.nFaces;
     c->nBF = d->sizes.nBoundaryFaces; c->nC = d->sizes.nCells;
@@ -1060,7 +1104,6 @@ extern "C" int adfvm_ctx_create(const adfvm_solver_desc* d, const adfvm_physics*
     c->phd.mu0 = ph->mu0; c->phd.muA = ph->muA; c->phd.muTs = ph->muTs; c->phd.muModel = ph->muModel;
     c->phd.riemann = ph->riemann; c->phd.boundaryRiemann = ph->boundaryRiemann;
     c->phd.limit = ph->limiter;
-    *out = c;
     if (c->nIC <= 0 || c->nF <= 0 || c->nBF < 0) return bad("bad mesh sizes");
     if (c->objective == ADFVM_OBJ_DRAG && (c->objectivePatch < 0 || c->objectivePatch >= c->nPatches))
         return bad("drag objective needs a valid patch index");
@@ -1097,20 +1140,20 @@ extern "C" int adfvm_ctx_create(const adfvm_solver_desc* d, const adfvm_physics*
         if (bPatch[b] < 0) return bad("boundary face not covered by a patch");
 
     // slot tables
-    std::vector<int> sFace(6 * nIC), sOther(6 * nIC), sPair(6 * nIC, -1);
-    std::vector<unsigned char> sFlags(6 * nIC);
-    std::vector<int> cellNb(6 * nIC);
-    for (long cc = 0; cc < nIC; cc++) {
+    std::vector<int> sPair(6 * nIC, -1);
+    Buffer<int> sFace(6 * nIC), sOther(6 * nIC), cellNb(6 * nIC);
+    Buffer<unsigned char> sFlags(6 * nIC);
+    auto slots_of = [&](long cc) -> const char* {         // the message where they are not valid
         for (int j = 0; j < 6; j++) {
             int f = d->cellFaces[6 * cc + j];
-            if (f < 0 || f >= nF) return bad("cellFaces out of range");
+            if (f < 0 || f >= nF) return "cellFaces out of range";
             int own = d->cellOwner[6 * cc + j];
             int other, kind;
             if (f < nIF) {
                 kind = SLOT_INTERNAL;
                 other = own ? d->neighbour[f] : d->owner[f];
             } else {
-                if (!own) return bad("boundary face in a neighbour slot");
+                if (!own) return "boundary face in a neighbour slot";
                 int b = f - nIF;
                 const adfvm_patch_desc& Pd = d->patches[bPatch[b]];
                 if (Pd.fluxKind == ADFVM_FLUX_COUPLED) {
@@ -1130,7 +1173,14 @@ extern "C" int adfvm_ctx_create(const adfvm_solver_desc* d, const adfvm_physics*
             sFlags[j * nIC + cc] = (unsigned char)((own ? 1 : 0) | (kind << 1) | (copy ? SLOT_GHOST_COPY : 0));
             cellNb[j * nIC + cc] = d->cellNeighbours[6 * cc + j];
         }
-    }
+        return nullptr;
+    };
+    std::vector<const char*> wrong(thread_parts((int)nIC, CELL_GRAIN), nullptr);
+    over_threads((int)nIC, CELL_GRAIN, [&](int first, int end, int part) {
+        for (long cc = first; cc < end && !wrong[part]; cc++) wrong[part] = slots_of(cc);
+    });
+    for (const char* w : wrong)
+        if (w) return bad(w);
     // face tables: the neighbour side's value source and the flux kind
     std::vector<int> fOther(nF);
     std::vector<unsigned char> fKind(nF);
@@ -1175,36 +1225,32 @@ extern "C" int adfvm_ctx_create(const adfvm_solver_desc* d, const adfvm_physics*
         if (posP[f] < 0) return bad("face without an owner slot");
         if (fKind[f] == FACE_INTERIOR && posN[f] < 0) return bad("face without a neighbour-side slot");
     }
-    int rc;
-    std::vector<int> owner(d->owner, d->owner + nF), nbFull(d->neighbour, d->neighbour + nF);
-    if ((rc = upload(c, (void**)&c->fOther, fOther)) != ADFVM_OK) return rc;
     for (long b = 0; b < nBF; b++)
         if (ghost_copies_owner(d->patches[bPatch[b]])) fKind[nIF + b] |= FACE_GHOST_COPY;
-    if ((rc = upload(c, (void**)&c->fKind, fKind)) != ADFVM_OK) return rc;
-    if ((rc = upload(c, (void**)&c->sFace, sFace)) != ADFVM_OK) return rc;
-    if ((rc = upload(c, (void**)&c->sOther, sOther)) != ADFVM_OK) return rc;
-    if ((rc = upload(c, (void**)&c->sFlags, sFlags)) != ADFVM_OK) return rc;
-    if ((rc = upload(c, (void**)&c->sPair, sPair)) != ADFVM_OK) return rc;
-    if ((rc = upload(c, (void**)&c->cellNbFull, cellNb)) != ADFVM_OK) return rc;
-    if ((rc = upload(c, (void**)&c->owner, owner)) != ADFVM_OK) return rc;
-    if ((rc = upload(c, (void**)&c->nbFull, nbFull)) != ADFVM_OK) return rc;
-    if ((rc = upload(c, (void**)&c->bPatch, bPatch)) != ADFVM_OK) return rc;
-    c->hBPatch = bPatch;
-    try {
+    // the tiles grow on a thread of their own while the other tables go to the
+    // device (a 24.7k-cell duct's context 5.4 -> 4.8 ms, 64^3 62 -> 48); on this one,
+    // at get(), where a thread is not to be had or would do little (1000 cells)
+    const auto policy = nIC < CELL_GRAIN ? std::launch::deferred : std::launch::async | std::launch::deferred;
+    std::future<Tiles> tiles = std::async(policy, [&] {
         Tiles t;
         build_tiles(TileMesh{(int)nIC, (int)nIF, (int)nF, sFace.data(), sOther.data(), sPair.data(), sFlags.data(),
                              fKind.data(), FACE_GHOST_COPY}, t);
-        c->nTiles = t.n;
-        if ((rc = upload(c, (void**)&c->toUser, t.toUser)) != ADFVM_OK) return rc;
-        if ((rc = upload(c, (void**)&c->toTile, t.toTile)) != ADFVM_OK) return rc;
-        if ((rc = upload(c, (void**)&c->tileFaceId, t.faceId)) != ADFVM_OK) return rc;
-        if ((rc = upload(c, (void**)&c->tilePairs, t.pairs)) != ADFVM_OK) return rc;
-        rc = c->prec == 4 ? create_typed<float>(c, d, t) : create_typed<double>(c, d, t);
-        if (rc != ADFVM_OK) return rc;
-    } catch (const std::exception& e) {
-        return bad(std::string("set-up of the mesh tables: ") + e.what());
-    }
-    if ((rc = upload(c, (void**)&c->patches, c->hpatches)) != ADFVM_OK) return rc;
+        return t;
+    });
+    int rc;
+    std::vector<int> owner(d->owner, d->owner + nF), nbFull(d->neighbour, d->neighbour + nF);
+    if ((rc = upload(c, &c->meshTables, {table(c->fOther, fOther), table(c->fKind, fKind), table(c->sFace, sFace),
+                                         table(c->sOther, sOther), table(c->sFlags, sFlags), table(c->sPair, sPair),
+                                         table(c->cellNbFull, cellNb), table(c->owner, owner), table(c->nbFull, nbFull),
+                                         table(c->bPatch, bPatch)})) != ADFVM_OK)
+        return rc;
+    c->hBPatch = bPatch;
+    rc = c->prec == 4 ? create_face_tables<float>(c, d) : create_face_tables<double>(c, d);
+    if (rc != ADFVM_OK) return rc;
+    const Tiles t = tiles.get();
+    c->nTiles = t.n;
+    rc = c->prec == 4 ? create_tile_tables<float>(c, d, t) : create_tile_tables<double>(c, d, t);
+    if (rc != ADFVM_OK) return rc;
     c->stream = stream_auto(c);
     c->nPartial = std::max(grid_bs(std::max<long>(nIC, nF), kBlockChoices[0]) + 1, c->nTiles);   // the smallest block size
     HIPCHK(c, hipMalloc((void**)&c->partial, 2L * c->nPartial * sizeof(double)));
@@ -1212,13 +1258,24 @@ extern "C" int adfvm_ctx_create(const adfvm_solver_desc* d, const adfvm_physics*
     return ADFVM_OK;
 }
 
+extern "C" int adfvm_ctx_create(const adfvm_solver_desc* d, const adfvm_physics* ph, adfvm_ctx** out) {
+    if (!d || !ph || !out) return ADFVM_ERR_INVALID;
+    *out = nullptr;
+    try {
+        *out = new adfvm_ctx();
+        return fill_context(*out, d, ph);
+    } catch (const std::exception& e) {
+        if (*out) (*out)->err = std::string("set-up of the mesh tables: ") + e.what();
+        return ADFVM_ERR_INVALID;
+    }
+}
+
 extern "C" void adfvm_ctx_destroy(adfvm_ctx* c) {
     if (!c) return;
-    void* ptrs[] = {c->geo, c->vol, c->bcval, c->sFace, c->sOther, c->sFlags, c->sPair, c->owner, c->bPatch,
-                    c->patches, c->cellNbFull, c->nbFull, c->ghost, c->st[0], c->st[1], c->st[2], c->rows1,
-                    c->rec[0], c->rec[1], c->rec[2], c->adjU, c->adjAcc, c->adjG,
-                    c->partial, c->scal, c->fOther, c->fKind, c->toUser, c->toTile, c->tileFaceId, c->tilePairs,
-                    c->tileBlock, c->tileRing, c->tileFaceW, c->segCell, c->segBlock, c->blockSeg, c->visc, c->ringCell, c->ringCount, c->ringCoef};
+    void* ptrs[] = {c->faceTables, c->meshTables, c->tileTables, c->ghost, c->st[0], c->st[1], c->st[2], c->rows1,
+                    c->rec[0], c->rec[1], c->rec[2], c->adjU, c->adjAcc, c->adjG, c->partial, c->scal, c->tileBlock,
+                    c->tileRing, c->tileFaceW, c->segTables, c->visc, c->ringCell, c->ringCount,
+                    c->ringCoef};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     for (auto& p : c->pending) { (void)hipEventDestroy(p.a); (void)hipEventDestroy(p.b); }
@@ -1282,13 +1339,10 @@ extern "C" int adfvm_set_segments(adfvm_ctx* c, int32_t nSeg, const int64_t* cel
         for (int b = 0; b < nb; b++) owner.push_back(k);
     }
     if (first[nSeg] > c->nPartial) return set_err(c, ADFVM_ERR_INVALID, "too many segment blocks");
-    for (void* p : {(void*)c->segCell, (void*)c->segBlock, (void*)c->blockSeg})
-        if (p) (void)hipFree(p);
-    c->segCell = nullptr; c->segBlock = nullptr; c->blockSeg = nullptr;
-    int rc;
-    if ((rc = upload(c, (void**)&c->segCell, cells)) != ADFVM_OK) return rc;
-    if ((rc = upload(c, (void**)&c->segBlock, first)) != ADFVM_OK) return rc;
-    if ((rc = upload(c, (void**)&c->blockSeg, owner)) != ADFVM_OK) return rc;
+    if (c->segTables) (void)hipFree(c->segTables);
+    c->segTables = nullptr; c->segCell = nullptr; c->segBlock = nullptr; c->blockSeg = nullptr;
+    const int rc = upload(c, &c->segTables, {table(c->segCell, cells), table(c->segBlock, first), table(c->blockSeg, owner)});
+    if (rc != ADFVM_OK) return rc;
     c->nSeg = nSeg;
     c->nSegBlocks = first[nSeg];
     return ADFVM_OK;
