@@ -47,3 +47,44 @@ def test_first_call_captured(prec):
         assert torch.equal(a, eager)
         eager.copy_(ua)
         ctx.adjoint_viscosity(u, eager, dt, 'abarbanel', scaling, iterations=20)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('n', [(40, 30, 1), (61, 60, 59)])
+@pytest.mark.parametrize('prec', [np.float32, np.float64])
+def test_alongside_steps_that_keep_tapes(n, prec):
+    """Sweeps on one stream while steps that keep their tapes run on another,
+    as in a reverse sweep that smooths the adjoint during a segment's re-run
+    (1200 cells, and 215940, whose steps convert rows): the bits of both in
+    turn."""
+    import torch
+    case = cf.CaseDef(meshgen.permute_and_rcm(meshgen.periodic_box(n), seed=5), {}, 1e-3)
+    ctx = case.context(prec)
+    u, ua, dt, scaling = _inputs(case, ctx)
+    steps = 8
+    tapes = ctx.new_tapes(steps)
+
+    def run_steps(v):
+        for k in range(steps):
+            ctx.primal_step(v, 1e-7, tape=tapes[k])
+
+    def smooth(a):
+        for _ in range(2):
+            ctx.adjoint_viscosity(u, a, dt, 'abarbanel', scaling, iterations=40)
+
+    v, a = u.clone(), ua.clone()
+    run_steps(v)
+    smooth(a)
+    kept = tapes.clone()
+    side = torch.cuda.Stream()
+    for _ in range(3):
+        v2, a2 = u.clone(), ua.clone()
+        tapes.zero_()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(side):
+            run_steps(v2)
+        smooth(a2)
+        torch.cuda.synchronize()
+        assert torch.equal(v2, v) and torch.equal(a2, a)
+        rows = 5 * ctx.nIC
+        assert torch.equal(tapes[:, :rows], kept[:, :rows])
