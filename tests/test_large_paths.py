@@ -1,0 +1,134 @@
+"""Meshes of more than 3072 tiles, whose steps turn the caller's rows into
+records and back: many copies of a small walled mesh side by side in one
+context, against the small mesh alone.  A cell's sums run over its own slots
+in order, so every copy has the small mesh's bits."""
+import copy
+import functools
+
+import numpy as np
+import pytest
+
+from adfvm_amd import _lib, meshgen
+from adfvm_amd.context import Context
+from adfvm_amd.mesh import Mesh
+from tests import casefactory as cf
+
+torch = pytest.importorskip('torch')
+pytestmark = pytest.mark.gpu
+
+N, COPIES = (13, 11, 9), 160                   # 1287 cells (21 tiles or more) and 205920 (3217 or more)
+
+
+def _small(cbc='CBC_UPT'):
+    c = cf.mixed_box(4, cbc, sutherland=True)
+    patches = {'x0': ('inlet', 'patch'), 'x1': ('outlet', 'patch'), 'y0': ('bottom', 'symmetryPlane'),
+               'y1': ('top', 'patch'), 'z0': ('sides', 'empty'), 'z1': ('sides', 'empty')}
+    md = meshgen.permute_and_rcm(meshgen.box(N, (1.3, 1.1, 0.9), patches=patches), seed=4)
+    rng = np.random.default_rng(4)
+    faces = N[1] * N[2]
+    c.bcs['inlet']['T']['value'] = 300 + rng.random((faces, 1))
+    c.bcs['outlet']['p']['p0'] = 1e5 + 10 * rng.random((faces, 1))
+    return md, c.bcs
+
+
+@functools.lru_cache(maxsize=None)
+def _meshes():
+    md, bcs = _small()
+    big, offsets = meshgen.concatenate([md] * COPIES, ['c%d_' % k for k in range(COPIES)])
+    all_bcs = {'c%d_%s' % (k, name): copy.deepcopy(spec) for k in range(COPIES) for name, spec in bcs.items()}
+    return (Mesh.from_data(md), bcs), (Mesh.from_data(big), all_bcs), offsets
+
+
+def _contexts(prec, integrator, objective):
+    """The small mesh's context and that of the copies; the drag is taken of the
+    first copy's top."""
+    (sm, sb), (bm, bb), _ = _meshes()
+    ph = dict(gamma=cf.GAMMA, Cp=cf.CP, Pr=cf.PR, mu=(_lib.MU_SUTHERLAND, 0., 1.4792e-06, 116.),
+              riemann=_lib.RIEMANN_ROE, boundaryRiemann=_lib.RIEMANN_ROE,
+              small=1e-30 if prec == np.float64 else 1e-9, integrator=integrator, objective=objective)
+    drag = objective == _lib.OBJ_DRAG
+    return (Context(sm, sb, dict(ph, **({'objectivePatch': 'top'} if drag else {})), prec),
+            Context(bm, bb, dict(ph, **({'objectivePatch': 'c0_top'} if drag else {})), prec))
+
+
+def _copies(a):
+    return a.repeat(1, COPIES).contiguous()
+
+
+def _run(ctx, u0, ua0, S, with_tape, mesh_grad):
+    f64 = lambda: torch.zeros(1, dtype=torch.float64, device='cuda')
+    u, ua, obj, dtc = u0.clone(), ua0.clone(), f64(), f64()
+    Sbar, bcg = torch.zeros_like(u0), ctx.bc_state()
+    mg = ctx.mesh_grad_state() if mesh_grad else None
+    tape = ctx.new_tapes(1)[0] if with_tape else None
+    ctx.profile_start()
+    ctx.primal_step(u, 1e-6, source=S, dtc_out=dtc, obj_out=obj, tape=tape)
+    ctx.adjoint_step(u0, 1e-6, ua, obja=0.7, source=S, source_grad=Sbar, bc_grad=bcg, tape=tape)
+    converted = 'to_records_kernel' in ctx.profile_stop()
+    return dict(u=u, ua=ua, Sbar=Sbar, bcg=bcg, obj=obj, dtc=dtc, mg=mg), converted
+
+
+@pytest.mark.parametrize('prec', [np.float32, np.float64])
+@pytest.mark.parametrize('with_tape', [False, True])
+@pytest.mark.parametrize('what', ['kinetic_energy', 'drag', 'start', 'euler', 'mesh_grad'])
+def test_copies_have_the_small_meshs_bits(prec, with_tape, what):
+    """State, adjoint, source and boundary-value gradients, time step limit:
+    bitwise.  Sums over all cells in FP64: 1e-12."""
+    integrator = _lib.RK_EULER if what == 'euler' else _lib.RK_SSPRK3
+    objective = _lib.OBJ_DRAG if what == 'drag' else _lib.OBJ_KINETIC_ENERGY
+    small, big = _contexts(prec, integrator, objective)
+    if what == 'start':
+        small.objective_state = big.objective_state = 'start'
+    case = cf.CaseDef(None, {}, 0.)
+    case._mesh = small.mesh
+    rng = np.random.default_rng(7)
+    u = cf.smooth_state(case, 4)
+    size = np.abs(u).mean(1, keepdims=True)
+    t = lambda a: torch.as_tensor(a.astype(prec), device='cuda').contiguous()
+    u0, ua0, S = t(u), t(rng.normal(size=u.shape) / size), t(0.01 * rng.normal(size=u.shape) * size)
+    one, converted = _run(small, u0, ua0, S, with_tape, what == 'mesh_grad')
+    assert not converted
+    all_, converted = _run(big, _copies(u0), _copies(ua0), _copies(S), with_tape, what == 'mesh_grad')
+    assert converted
+    objective_copies = 1 if what == 'drag' else COPIES      # the copies that the objective is taken of
+    if what == 'drag':
+        rest, _ = _run(_contexts(prec, integrator, _lib.OBJ_NONE)[0], u0, ua0, S, with_tape, False)
+    n = small.nIC
+    for k in range(COPIES):
+        ref = one if k < objective_copies else rest
+        for name in ('u', 'ua', 'Sbar'):
+            assert torch.equal(all_[name][:, k * n:(k + 1) * n], ref[name]), (name, k)
+    # boundary faces: copy after copy, patches in the same order
+    per = all_['bcg'].reshape(5, COPIES, small.nBF)
+    for k in range(COPIES):
+        assert torch.equal(per[:, k], (one if k < objective_copies else rest)['bcg']), k
+    assert torch.equal(all_['dtc'], one['dtc'])
+    assert abs(all_['obj'].item() - objective_copies * one['obj'].item()) <= 1e-12 * abs(all_['obj'].item())
+    if what == 'mesh_grad':
+        nIF, nBF = small.mesh.nInternalFaces, small.nBF
+        for a, b in zip(big.mesh_grad_arrays(all_['mg']), small.mesh_grad_arrays(one['mg'])):
+            rows = len(b)
+            if rows == n or rows == nIF:
+                assert torch.equal(a.reshape((COPIES,) + b.shape), b.expand((COPIES,) + b.shape))
+            else:
+                inner, outer = a[:COPIES * nIF], a[COPIES * nIF:]
+                assert torch.equal(inner.reshape((COPIES, nIF) + b.shape[1:]), b[:nIF].expand((COPIES, nIF) + b.shape[1:]))
+                assert torch.equal(outer.reshape((COPIES, nBF) + b.shape[1:]), b[nIF:].expand((COPIES, nBF) + b.shape[1:]))
+
+
+@pytest.mark.parametrize('prec', [np.float32, np.float64])
+def test_objective_of_each_copy(prec):
+    """The copies as segments: each copy's kinetic energy has the small mesh's
+    bits."""
+    small, big = _contexts(prec, _lib.RK_SSPRK3, _lib.OBJ_KINETIC_ENERGY)
+    big.set_segments(_meshes()[2])
+    small.set_segments([0, small.nIC])
+    case = cf.CaseDef(None, {}, 0.)
+    case._mesh = small.mesh
+    u0 = torch.as_tensor(cf.smooth_state(case, 4).astype(prec), device='cuda').contiguous()
+    J1 = torch.zeros(1, dtype=torch.float64, device='cuda')
+    J = torch.zeros(COPIES, dtype=torch.float64, device='cuda')
+    u, v = u0.clone(), _copies(u0)
+    small.primal_step(u, 1e-6, obj_out=J1)
+    big.primal_step(v, 1e-6, obj_out=J)
+    assert torch.equal(v, _copies(u)) and torch.equal(J, J1.expand(COPIES))

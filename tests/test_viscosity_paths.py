@@ -88,3 +88,39 @@ def test_alongside_steps_that_keep_tapes(n, prec):
         assert torch.equal(v2, v) and torch.equal(a2, a)
         rows = 5 * ctx.nIC
         assert torch.equal(tapes[:, :rows], kept[:, :rows])
+
+
+# tiles a patch, and whether several sweeps a launch pay
+PATCHES = {
+    'o_grid_2_tiles': (lambda: meshgen.o_grid(160, 130), True),
+    'o_grid_5_tiles': (lambda: meshgen.o_grid(301, 261), True),
+    'walls_2_tiles': (lambda: meshgen.permute_and_rcm(meshgen.box((31, 30, 29)), seed=5), True),
+    'box_above_limit': (lambda: meshgen.permute_and_rcm(meshgen.periodic_box((64, 63, 62)), seed=5), False),
+}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('name', sorted(PATCHES))
+@pytest.mark.parametrize('prec', [np.float32, np.float64])
+@pytest.mark.parametrize('iterations', [2, 37])
+def test_patches_of_several_tiles(name, prec, iterations):
+    """Patches of 2 and 5 tiles, the last one smaller than the others, with and
+    without ghosts, and a mesh whose rings do not fit: the sweeps of a captured
+    first call, one at a time, against those of a call outside a capture."""
+    import torch
+    make, several = PATCHES[name]
+    case = cf.CaseDef(make(), {}, 1e-3)
+    ctx = case.context(prec)
+    u, ua, dt, scaling = _inputs(case, ctx)
+    one = ua.clone()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, capture_error_mode='relaxed'):
+        ctx.adjoint_viscosity(u, one, dt, 'abarbanel', scaling, iterations=iterations)
+    graph.replay()
+    many = ua.clone()
+    kernels = _sweep_kernels(ctx, lambda: ctx.adjoint_viscosity(u, many, dt, 'abarbanel', scaling,
+                                                                iterations=iterations))
+    assert list(kernels) == (['visc_rings_kernel'] if several else ['visc_jacobi_kernel'])
+    assert torch.isfinite(many).all() and not torch.equal(many, ua)
+    assert torch.equal(one, many)
