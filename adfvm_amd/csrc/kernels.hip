@@ -648,9 +648,9 @@ int grid_for(long n) { return (int)((n + BLOCK - 1) / BLOCK); }
 int grid_bs(long n, int bs) { return (int)((n + bs - 1) / bs); }
 
 // The stencil kernels' names and the block sizes adfvm_set_kernel_block
-// takes.  A tile fixes the block at TILE_THREADS (one thread per face of the
-// tile); the flux and the stage update, and the face adjoint and its gather,
-// are one kernel each.
+// takes.  A tile fixes the blocks: TILE_CELLS threads (one per cell) for the
+// gradient and its transpose, else TILE_THREADS (one per face); the flux and the
+// stage update, and the face adjoint and its gather, are one kernel each.
 enum { K_GRAD = 0, K_FLUX, K_STAGE, K_FVJP, K_GATHER, K_GVJP, K_TUNABLE };
 const char* const kTunableName[K_TUNABLE] = {"grad_kernel", "face_flux_kernel", "stage_kernel",
                                               "face_vjp_kernel", "vjp_gather_kernel", "grad_vjp_kernel"};

@@ -335,8 +335,9 @@ int adfvm_adjoint_viscosity(adfvm_ctx* ctx, const void* u_n, void* ua, double dt
  * so it is not for use inside graph capture.  No counterpart in the reference
  * (adpy fixes its launch shapes at code generation). */
 int adfvm_autotune(adfvm_ctx* ctx, const void* u, int32_t reps, void* stream);
-/* i-th stencil kernel name (0 <= i < 6), its block size (256) and the time per
- * launch adfvm_autotune measured for it (-1 before). */
+/* i-th stencil kernel name (0 <= i < 6), its block size (64 for grad_kernel and
+ * grad_vjp_kernel, 256 for the others) and the time per launch adfvm_autotune
+ * measured for it (-1 before). */
 int adfvm_kernel_config(const adfvm_ctx* ctx, int32_t i, char* name, int32_t len, int32_t* block,
                         double* ms);
 /* Accepts a block size (64, 128, 256 or 512) for a stencil kernel's name; the

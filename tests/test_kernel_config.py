@@ -1,0 +1,30 @@
+"""What the library reports of its stencil kernels: the blocks they launch."""
+import numpy as np
+import pytest
+
+from tests import casefactory as cf
+
+BLOCKS = {'grad_kernel': 64, 'face_flux_kernel': 256, 'stage_kernel': 256, 'face_vjp_kernel': 256,
+          'vjp_gather_kernel': 256, 'grad_vjp_kernel': 64}
+
+
+@pytest.mark.gpu
+def test_reported_blocks():
+    """A tile's cells for the gradient and its transpose, a tile's faces for the
+    others; before and after a size is set (accepted, without effect) and the
+    kernels are timed.  Names and sizes that were never taken are refused."""
+    import torch
+    case, params = cf.tgv(6)
+    ctx = case.context(np.float32)
+    blocks = lambda: {k: b for k, (b, _) in ctx.kernel_config().items()}
+    assert blocks() == BLOCKS
+    for k in BLOCKS:
+        for b in (64, 128, 256, 512):
+            ctx.set_kernel_block(k, b)
+    assert blocks() == BLOCKS
+    u = torch.as_tensor(cf.tgv_state(case, params).astype(np.float32), device='cuda').contiguous()
+    assert all(ms > 0 for _, ms in ctx.autotune(u, reps=1).values())
+    assert blocks() == BLOCKS
+    for k, b in (('grad_kernel', 96), ('tile_stage_kernel', 64)):
+        with pytest.raises(Exception):
+            ctx.set_kernel_block(k, b)
