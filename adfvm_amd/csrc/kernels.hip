@@ -93,24 +93,19 @@ template <typename T> struct DMesh {
     const T* bcval;
 };
 
-// Loads and stores of data a launch touches once, in rows whose cache lines
-// one instruction consumes whole (face geometry, slot tables, a thread's own
-// state rows): non-temporal, so that they are first out of L2 and the cell
-// records that neighbouring threads read again stay in it (grad 6%, face
-// flux 5%, gradient adjoint 8% faster at TGV 128^3 FP32).  Not for records
-// that straddle lines or that lanes share: there the hint re-fetches lines
-// (adjoint gather 55% slower with non-temporal record loads).
-// ST selects it per context (adfvm_ctx::stream): on meshes whose stage
-// working set fits the 256 MB Infinity Cache the same rows are reused by the
-// next kernels and stages, and plain loads keep them there (the 512 x 256
-// cylinder ran 9% slower streamed).
+// Loads of data a launch touches once, in pieces whose cache lines one
+// instruction consumes whole (a tile's tables and geometry; ldp the same in 16
+// bytes): non-temporal, so that they are first out of L2 and the records that
+// neighbouring tiles read again stay in it (128^3 FP32 step 907 -> 802 us).  Not for
+// records that straddle lines or that lanes share: there the hint re-fetches
+// lines.
+// ST selects it per context (adfvm_ctx::stream): on meshes whose stage works on
+// less than the 256 MB Infinity Cache the next kernels and stages find the same
+// tables there, and plain loads keep them (a 64^3 FP32 step takes 119 us
+// streamed, 108 not).
 template <bool ST, typename T> __device__ __forceinline__ T ld(const T* p) {
     if constexpr (ST) return __builtin_nontemporal_load(p);
     else return *p;
-}
-template <bool ST, typename T> __device__ __forceinline__ void st(T* p, T v) {
-    if constexpr (ST) __builtin_nontemporal_store(v, p);
-    else *p = v;
 }
 
 // Geometry of face f.
@@ -671,16 +666,18 @@ template <typename F> void with_ghosts(bool gh, F&& f) {
     else f(std::bool_constant<false>());
 }
 
-// The automatic streaming policy: on when one RK stage's working set
-// exceeds the 256 MB Infinity Cache.  Per face: 17 geometry rows, the face
-// tables (9 B) and a flux record (8 scalars); per cell: state, gradient
-// record, slot geometry, volume, three stage states (61 scalars) and the
-// slot tables (30 B).
-bool stream_auto(const adfvm_ctx* c) {
-    const double s = c->prec;
-    const double bytes = (double)c->nF * (25 * s + 9) + (double)c->nIC * (61 * s + 30);
-    return bytes > 256.0 * (1 << 20);
+// The automatic streaming policy: on when what a stage works on exceeds the
+// 256 MB Infinity Cache: the tiles' blocks, the stage records and three states
+// (the stage's, the step's start and the next).  Off -> on, steps in us: 268 MB (80^3
+// FP32) 210 -> 213, with their adjoint steps 495 -> 490; 458 MB (96^3) 366 -> 339 and 850
+// -> 803; 228 MB (410k cells of an O-grid) 178 -> 185 and 421 -> 428; FP64 263 MB
+// (64^3) 225 -> 232 and 573 -> 569; 375 MB (72^3) 316 -> 304 and 793 -> 771; 215 MB (a
+// 60^3 duct) 252 -> 261 and 575 -> 580.
+template <typename T> bool stream_auto(const adfvm_ctx* c) {
+    const double tile = TileBlock<T>::BYTES + (CREC + 15.0) * TILE_CELLS * sizeof(T);
+    return c->nTiles * tile > 256.0 * (1 << 20);
 }
+bool stream_auto(const adfvm_ctx* c) { return c->prec == 4 ? stream_auto<float>(c) : stream_auto<double>(c); }
 
 template <typename T> Phys<T> phys_cast(const Phys<double>& p) {
     Phys<T> o;

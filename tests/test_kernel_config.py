@@ -1,7 +1,9 @@
-"""What the library reports of its stencil kernels: the blocks they launch."""
+"""What the library reports of its stencil kernels: the blocks they launch and
+the automatic streaming policy."""
 import numpy as np
 import pytest
 
+from adfvm_amd import meshgen
 from tests import casefactory as cf
 
 BLOCKS = {'grad_kernel': 64, 'face_flux_kernel': 256, 'stage_kernel': 256, 'face_vjp_kernel': 256,
@@ -28,3 +30,17 @@ def test_reported_blocks():
     for k, b in (('grad_kernel', 96), ('tile_stage_kernel', 64)):
         with pytest.raises(Exception):
             ctx.set_kernel_block(k, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('make,prec,want', [
+    (lambda: meshgen.o_grid(800, 512), np.float32, False),          # 211 MB or more
+    (lambda: meshgen.periodic_box((80, 80, 80)), np.float32, True),      # 264 MB or more
+    (lambda: meshgen.o_grid(520, 400), np.float64, False),          # 206 MB or more
+    (lambda: meshgen.o_grid(800, 512), np.float64, True),           # 405 MB or more
+])
+def test_automatic_streaming(make, prec, want):
+    """On where a tile's block, 20 record scalars and 15 state scalars per cell
+    come to more than 256 MB over the tiles (a mesh of n cells has n/64 or a few
+    percent more)."""
+    assert cf.CaseDef(make(), {}, 1e-3).context(prec).streaming is want
