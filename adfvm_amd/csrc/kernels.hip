@@ -38,10 +38,10 @@ using namespace adfvm;
 
 // Workgroups of a launch are dealt to the 8 XCDs round-robin (block b runs
 // on XCD b % 8), and each XCD has its own L2.  The stencil kernels remap
-// block b to a logical block so that every XCD works through one contiguous
-// eighth of the cells (or faces): the neighbours a block gathers (RCM
-// order: within a few thousand rows) were then recently touched on the
-// same XCD and hit its L2.  The map is a bijection of [0, gridDim.x).
+// block b to a tile so that every XCD works through one contiguous eighth of
+// the tiles: those it works on at one time lie near one another in the mesh
+// (order_tiles), and a tile's halo is in its L2 as its neighbours' own cells.
+// The map is a bijection of [0, gridDim.x).
 __device__ __forceinline__ int xcd_block() {
     const unsigned nb = gridDim.x, b = blockIdx.x;
     const unsigned q = nb >> 3, r = nb & 7u, x = b & 7u, k = b >> 3;
@@ -49,15 +49,13 @@ __device__ __forceinline__ int xcd_block() {
 }
 
 // ------------------------------------------------------------- tables ----
-// slot flags: bit 0 = this cell owns the face; bits 1-2 = slot kind; bit 3
-// (boundary slots) = the ghost's values are the owner's (zeroGradient U, and
-// zeroGradient or symmetry T and p: BCs.py:97-104,120-137), so neither the
-// ghost rule nor its adjoint needs the patch
+// slot flags: bit 0 = this cell owns the face; bits 1-2 = slot kind
 enum { SLOT_INTERNAL = 0, SLOT_COUPLED = 1, SLOT_CHARACTERISTIC = 2, SLOT_BOUNDARY = 3 };
-constexpr int SLOT_GHOST_COPY = 8;
 __host__ __device__ __forceinline__ int slot_kind(int flags) { return (flags >> 1) & 3; }
 // face kind bytes (device copy): FACE_* in bits 0-1, bit 2 for a boundary
-// face whose ghost copies its owner (as the slot flag above)
+// face whose ghost's values are the owner's (zeroGradient U, and zeroGradient or
+// symmetry T and p: BCs.py:97-104,120-137), so that neither the ghost rule nor its
+// adjoint needs the patch
 constexpr int FACE_GHOST_COPY = 4;
 __host__ __device__ __forceinline__ int face_kind(int k) { return k & 3; }
 
@@ -87,7 +85,7 @@ template <typename T> struct DMesh {
     const int* sPair;       // [6][nIC]: paired face of a coupled slot, else -1
     const int* owner;       // [nF]
     const int* fOther;      // [nF]: neighbour, paired internal cell (cyclic) or -1-b (ghost)
-    const unsigned char* fKind;  // [nF]: FACE_INTERIOR / FACE_CHARACTERISTIC / FACE_BOUNDARY
+    const unsigned char* fKind;  // [nF]: face kind bytes
     const int* bPatch;      // [nBF]
     const DPatch* patches;
     const T* bcval;
@@ -528,12 +526,6 @@ __global__ void fill_kernel(double* p, int n, double v) {
     if (i < n) p[i] = v;
 }
 
-template <typename T>
-__global__ void __launch_bounds__(BLOCK) copy_kernel(long n, const T* __restrict__ x, T* __restrict__ y) {
-    long i = (long)blockIdx.x * BLOCK + threadIdx.x;
-    if (i < n) y[i] = x[i];
-}
-
 // ----------------------------------------------------------- context -----
 
 struct adfvm_ctx {
@@ -690,7 +682,7 @@ template <typename T> Phys<T> phys_cast(const Phys<double>& p) {
 template <typename T> DMesh<T> dmesh(const adfvm_ctx* c) {
     DMesh<T> m;
     m.nIC = c->nIC; m.nIF = c->nIF; m.nF = c->nF; m.nBF = c->nBF;
-    m.geo = (const T*)c->geo; m.vol = (const T*)c->vol; 
+    m.geo = (const T*)c->geo; m.vol = (const T*)c->vol;
     m.sFace = c->sFace; m.sOther = c->sOther; m.sFlags = c->sFlags; m.sPair = c->sPair;
     m.owner = c->owner; m.bPatch = c->bPatch; m.patches = c->patches; m.bcval = (const T*)c->bcval;
     m.fOther = c->fOther; m.fKind = c->fKind;
@@ -1166,8 +1158,7 @@ static int fill_context(adfvm_ctx* c, const adfvm_solver_desc* d, const adfvm_ph
             }
             sFace[j * nIC + cc] = f;
             sOther[j * nIC + cc] = other;
-            const bool copy = kind == SLOT_BOUNDARY && ghost_copies_owner(d->patches[bPatch[f - nIF]]);
-            sFlags[j * nIC + cc] = (unsigned char)((own ? 1 : 0) | (kind << 1) | (copy ? SLOT_GHOST_COPY : 0));
+            sFlags[j * nIC + cc] = (unsigned char)((own ? 1 : 0) | (kind << 1));
             cellNb[j * nIC + cc] = d->cellNeighbours[6 * cc + j];
         }
         return nullptr;

@@ -16,9 +16,9 @@ segment -- is one captured graph, replayed as a single launch per sweep.
 
 With overlap (the default when a second set of segment buffers fits in
 device memory), the re-run of segment s-1 goes on a second stream while the
-adjoint steps of segment s run: the two use separate stage-state and tape
-buffers and disjoint context work buffers (the primal's face-flux records,
-the adjoint's face and cell adjoint records), and events order each re-run
+adjoint steps of segment s run: the two use separate start-state and tape
+buffers and disjoint context work buffers (the primal's stage states, the
+adjoint's states and cell adjoint records), and events order each re-run
 after the adjoint steps that last read its buffers and before the adjoint
 steps that read them next.  Every kernel computes what it computed in
 sequence: the results are bit-identical.

@@ -38,8 +38,9 @@ def kernel_bytes(name, s, nC, nF, nG, nO=None):
     records (5 primitives, 15 gradients), cell adjoint records (15 + 5) and,
     per tile of about 64 cells, the geometry of its faces (16 rows, 4 B of
     indices) or of its cells' slots (24 values), 24 B of indices per cell.
-    face_vjp_kernel and vjp_gather_kernel are a face kernel writing face
-    adjoint records (20 scalars) and the gather of them into cells: with nO
+    face_vjp_kernel and vjp_gather_kernel, which the library does not have, are
+    what flux_vjp_kernel does in one launch as two: a face kernel writing face
+    adjoint records (20 scalars) and the gather of them into cells.  With nO
     cells owning internal faces (owner sides summed per cell) one record per
     internal face, one per such cell and two per cyclic face, otherwise two
     per face (nO None); record indices (int32) 4 B per record written by face,
@@ -430,9 +431,6 @@ def main():
     m = case.mesh
     nC, nF = m.nInternalCells, m.nFaces
     nG = m.nFaces - m.nInternalFaces
-    own = np.asarray(m.owner[:m.nInternalFaces])
-    # the face adjoint sums owner sides per cell when internal faces are in owner order
-    nO = len(np.unique(own)) if np.all(np.diff(own) >= 0) else None
     u0 = cf.tgv_state(case, params)
     dx = 2 * np.pi / args.n
     c0 = np.sqrt(cf.GAMMA * cf.R * params['T0'])
@@ -461,7 +459,7 @@ def main():
     dom = max(prof, key=lambda k: prof[k][0])
     ms_tot, launches = prof[dom]
     avg_s = ms_tot / launches * 1e-3
-    kb = kernel_bytes(dom, 4, nC, nF, nG, nO)
+    kb = kernel_bytes(dom, 4, nC, nF, nG)
     achieved = kb / avg_s / 1e9 if kb else None
     traffic = None
     tf = os.path.join(ROOT, 'profiles', 'traffic.json')
@@ -486,7 +484,7 @@ def main():
         'config': {'workload': 'TGV %d^3 periodic hex, random permutation + RCM, primal+adjoint, SSP-RK3, Roe, '
                                'fixed dt, start states and step tapes (stage states + gradients) of all K steps '
                                'kept in HBM' % args.n,
-                   'n_cells': nC, 'n_faces': nF, 'n_owner_records': nO, 'dt': dt,
+                   'n_cells': nC, 'n_faces': nF, 'dt': dt,
                    'objective': 'kinetic energy on the stage-1 state'},
         'roofline': {'bound': 'hbm', 'kernel': dom, 'achieved': achieved, 'peak': HBM_PEAK / 1e9, 'unit': 'GB/s',
                      'frac': (achieved / (HBM_PEAK / 1e9)) if achieved else None, 'traffic': traffic,
@@ -498,7 +496,7 @@ def main():
         'primal_cell_updates_per_s_fp32': nC * K / r32['t_p'],
         'value_fp32_recompute_stages': nC * K / r32r['t_pa'] if r32r else None,
         'kernel_ms_fp32': {k: round(v[0] / K, 4) for k, v in prof.items()},
-        'kernel_roofline_fp32': kernel_rooflines(prof, 4, nC, nF, nG, nO, triad),
+        'kernel_roofline_fp32': kernel_rooflines(prof, 4, nC, nF, nG, None, triad),
         'block_sizes_fp32': r32['tuned'],
         'streaming_fp32': r32['streaming'],
         'finite': r32['finite'],
