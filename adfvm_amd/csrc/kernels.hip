@@ -258,11 +258,14 @@ __device__ void block_reduce_store(double v, double* out) {
 
 // A thread's share of n partials, those at its index and every THREADS-th after
 // it, folded in order.  Loads in batches of 32: one block waits for each batch,
-// and nothing else runs meanwhile (a load at a time, 33k partials took 44 us).
+// and nothing else runs meanwhile (a load at a time, 33k partials took 44 us); one
+// partial a thread skips the rest of its batch (a 1000-cell FP64 step 32.9 -> 31.7
+// us).
 template <int OP, int THREADS>
 __device__ __forceinline__ double fold_partials(const double* __restrict__ partials, int n) {
     constexpr int BATCH = 32;
     const double none = OP == 0 ? 0.0 : -1.0e308;
+    if (n <= THREADS) return combine<OP>(none, (int)threadIdx.x < n ? partials[threadIdx.x] : none);
     double v = none;
     for (int i = threadIdx.x; i < n; i += BATCH * THREADS) {
         double x[BATCH];
