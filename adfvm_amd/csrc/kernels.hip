@@ -877,14 +877,14 @@ template <typename T> void launch_ghosts(adfvm_ctx* c, const T* u, hipStream_t s
     ghost_kernel<T><<<grid_for(c->nBF), BLOCK, 0, s>>>(dmesh<T>(c), phys_cast<T>(c->phd), u, P<T>(c->ghost));
 }
 
-// Stage records of state u: the caller's rows (user) or state records; copy
-// (nullable): u as state records.
-template <typename T> void launch_grad(adfvm_ctx* c, const T* u, bool user, T* copy, T* rec, hipStream_t s) {
+// Stage records (GONLY: gradients alone) of state u: the caller's rows (user) or
+// state records; copy (nullable): u as state records.
+template <typename T, bool GONLY = false> void launch_grad(adfvm_ctx* c, const T* u, bool user, T* copy, T* rec, hipStream_t s) {
     KTimer kt(c, "grad_kernel", s);
     with_stream(c->stream, [&](auto SP) {
         with_ghosts(c->hasGhostKernel, [&](auto G) {
             constexpr bool ST = decltype(SP)::value, GH = decltype(G)::value;
-            grad_kernel<T, ST, GH><<<c->nTiles, TILE_CELLS, 0, s>>>(dmesh<T>(c), dtiles<T>(c),
+            grad_kernel<T, ST, GH, GONLY><<<c->nTiles, TILE_CELLS, 0, s>>>(dmesh<T>(c), dtiles<T>(c),
                                                                       phys_cast<T>(c->phd), u, user, copy, rec);
         });
     });
@@ -1363,7 +1363,12 @@ extern "C" int adfvm_primal_step(adfvm_ctx* c, void* u, double dt, const void* S
 
 namespace {
 template <typename T> int gradients_t(adfvm_ctx* c, const T* u, T* grad, hipStream_t s) {
-    launch_grad<T>(c, u, true, nullptr, P<T>(c->rec[0]), s);
+    // as steps do, but in a buffer that steps with a tape do not use.  100^3 FP32
+    // 88.5 us on the rows, 71 with the conversion; 64^3 24.8 and 23.9 (FP64 41.3 and
+    // 41.1); O-grids of longer runs 30 and 32 (410k cells)
+    const bool convert = converts_rows(c);
+    if (convert) launch_to_records<T>(c, u, P<T>(c->rec[1]), s);
+    launch_grad<T, true>(c, convert ? P<T>(c->rec[1]) : u, !convert, nullptr, P<T>(c->rec[0]), s);
     grad_rows_kernel<T><<<grid_for(c->nIC), BLOCK, 0, s>>>(dtiles<T>(c), c->nIC, P<T>(c->rec[0]), grad);
     HIPCHK(c, hipGetLastError());
     return ADFVM_OK;

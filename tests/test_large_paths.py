@@ -132,3 +132,22 @@ def test_objective_of_each_copy(prec):
     small.primal_step(u, 1e-6, obj_out=J1)
     big.primal_step(v, 1e-6, obj_out=J)
     assert torch.equal(v, _copies(u)) and torch.equal(J, J1.expand(COPIES))
+
+
+@pytest.mark.parametrize('prec', [np.float32, np.float64])
+def test_operators_of_copies(prec):
+    """Gradients, the residual with its eigenvalue sums, and the residual's
+    transpose: every copy has the small mesh's bits."""
+    small, big = _contexts(prec, _lib.RK_SSPRK3, _lib.OBJ_NONE)
+    case = cf.CaseDef(None, {}, 0.)
+    case._mesh = small.mesh
+    u = cf.smooth_state(case, 4)
+    t = lambda a: torch.as_tensor(a.astype(prec), device='cuda').contiguous()
+    u0, b0 = t(u), t(np.random.default_rng(7).normal(size=u.shape) / np.abs(u).mean(1, keepdims=True))
+
+    def run(ctx, u, b):
+        dtc = torch.zeros(ctx.nIC, dtype=ctx.tdtype, device='cuda')
+        return [ctx.gradients(u).reshape(15, -1), ctx.residual(u, dtc_cell=dtc), dtc[None], ctx.residual_vjp(u, b)]
+
+    for one, all_ in zip(run(small, u0, b0), run(big, _copies(u0), _copies(b0))):
+        assert torch.equal(all_, _copies(one))
