@@ -147,9 +147,13 @@ class Solver(object):
                 dt = float(dts[timeIndex]) if timeIndex < len(dts) else dt
             elif not fixed:
                 limit = dtc.item()
-                if limit != limit:       # no next dt: min() below would return NaN and end the loop silently
-                    raise FloatingPointError('NaN in the time step limit at step %d (t=%g)' % (timeIndex, t))
-                dt = min(2 * self.CFL / limit, dt * self.stepFactor, endTime - t)
+                if limit == limit:
+                    dt = min(2 * self.CFL / limit, dt * self.stepFactor, endTime - t)
+                elif not bool(torch.isfinite(self.u).all()):
+                    # no next dt: min() would return NaN and end the loop silently
+                    raise FloatingPointError('NaN/Inf in the state at step %d (t=%g)' % (timeIndex, t))
+                else:                    # a face's eigenvalue alone is no number: the step stays
+                    dt = min(dt, endTime - t)
             if write and mode != 'forward':
                 if mode in ('orig', 'simulation'):
                     self.writeFields(t)

@@ -48,3 +48,21 @@ def test_run_with_time_step_control_stops(n):
     with pytest.raises(FloatingPointError):
         s.run(endTime=1.0, dt=1e-6, nSteps=5, reportInterval=1000, mode='forward')
     config.set_precision(precision)
+
+
+@pytest.mark.gpu
+def test_run_goes_on_with_a_finite_state(monkeypatch):
+    """A limit that is NaN beside a finite state (an eigenvalue of a
+    reconstructed face value alone) keeps the step."""
+    case, params = cf.tgv(5)
+    precision = config.precision
+    s = cf.rcf(case, cf.tgv_state(case, params), np.float64, CFL=0.5, stepFactor=1.2)
+    step = s.step
+
+    def with_nan(u, dt, source, dtc_out, obj_out, tape=None):
+        step(u, dt, source, dtc_out, obj_out, tape)
+        dtc_out.fill_(float('nan'))
+    monkeypatch.setattr(s, 'step', with_nan)
+    states = s.run(endTime=1.0, dt=1e-6, nSteps=3, reportInterval=1, mode='forward')
+    config.set_precision(precision)
+    assert len(states) == 4 and s.lastDt == 1e-6 and s.lastTime == 3e-6
